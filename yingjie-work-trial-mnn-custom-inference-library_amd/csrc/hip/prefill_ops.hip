@@ -647,9 +647,13 @@ static size_t gemm_prep_bytes(int m, int cols) {
            m_pad * static_cast<size_t>(cols / 64) * sizeof(float) + m_pad * sizeof(float);
 }
 
+// A bound that grows with m and with rows, so that a workspace sized for a
+// chunk's most tokens and widest matrix serves every smaller call: the partial
+// products of a split launch (fewer tokens or rows can split into more) never
+// exceed kGemmMaxSplits m rows, nor the tiles of fewer than 2 x 512 blocks.
 size_t gemm_workspace_bytes(int m, int cols, int rows) {
-    const int splits = rows > 0 ? gemm_splits(rows, m, cols, 0) : 1;
-    const size_t part = splits > 1 ? static_cast<size_t>(splits) * m * rows * sizeof(float) : 0;
+    const size_t all = static_cast<size_t>(kGemmMaxSplits) * m * std::max(0, rows);
+    const size_t part = std::min<size_t>(all, size_t{2 * 512} * kGemmBR * kGemmBT) * sizeof(float);
     return gemm_prep_bytes(m, cols) + (part + 255) / 256 * 256;
 }
 
