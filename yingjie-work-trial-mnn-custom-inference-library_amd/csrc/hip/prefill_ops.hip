@@ -12,7 +12,6 @@
 //                        x hi / lo on v_mfma_f32_16x16x32_f16, group sums scaled
 //                        by the group scale; the zero-point term as a K = G
 //                        MFMA contraction after the group loop
-//   prefill_attn_mfma_kernel / prefill_attn_kernel   causal GQA over the cache
 //   linear_conv_prefill_tg_kernel + scan_chunk_prep_kernel + scan_chunk_state_kernel   conv1d + norms +
 //                        gates for all tokens, then the gated-delta recurrence
 //                        with the state in registers (one-pass kernels
@@ -742,293 +741,6 @@ hipError_t launch_gemm(const GemmLaunch& p, hipStream_t s) {
     const int blocks = static_cast<int>(std::min<size_t>((n + 255) / 256, 2048));
     hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3(blocks), dim3(256), 0, s, part, splits, p.m, p.rows, p.y,
                        p.ldy, p.epi == 1 ? 1 : 0);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Causal GQA for a prompt chunk: block (t, kh) takes query token t (position
-// pos0 + t) and the `group` query heads of kv head kh over keys 0..pos0+t in
-// 64-token chunks with a running max / sum (rescaled by exp(m_old - m_new)),
-// then normalises by multiplying with 1/l and applies the sigmoid gate
-// (custom_model.cpp:840-951 per token).
-// ---------------------------------------------------------------------------
-constexpr int kPAttnChunk = 64;
-constexpr int kPAttnMaxGroup = 8;
-
-__global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) {
-    extern __shared__ float smem[];
-    const int t = blockIdx.x, kh = blockIdx.y;
-    const int hd = p.head_dim, group = p.nq / p.nkv;
-    const int ctx = *p.pos0 + t + 1;
-    float* qs = smem;                        // [group][hd]
-    float* sc = qs + group * hd;             // [group][64]
-    float* osum = sc + group * kPAttnChunk;  // [group][hd] running output
-    float* ml = osum + group * hd;           // [group][2] running max, sum
-    float* fac = ml + 2 * group;             // [group] rescale of this chunk
-    const float* qrow = p.q + static_cast<size_t>(t) * p.q_stride + static_cast<size_t>(kh) * group * hd;
-    for (int i = threadIdx.x; i < group * hd; i += blockDim.x) {
-        qs[i] = qrow[i];
-        osum[i] = 0.0f;
-    }
-    if (threadIdx.x < group) {
-        ml[2 * threadIdx.x] = -INFINITY;
-        ml[2 * threadIdx.x + 1] = 0.0f;
-    }
-    __syncthreads();
-    const float rscale = 1.0f / sqrtf(static_cast<float>(hd));
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    for (int c0 = 0; c0 < ctx; c0 += kPAttnChunk) {
-        const int n = min(kPAttnChunk, ctx - c0);
-        // scores: 4 threads per key, each a quarter of the dims
-        {
-            const int sub = threadIdx.x & 3, tt = threadIdx.x >> 2;
-            const int dq = (hd + 3) / 4, d0 = sub * dq, d1 = min(hd, d0 + dq);
-            const bool valid = tt < n;
-            const _Float16* krow = p.k_cache + (static_cast<size_t>(c0 + (valid ? tt : 0)) * p.nkv + kh) * hd;
-            for (int g = 0; g < group; ++g) {
-                float dot = 0.0f;
-                for (int d = d0; d < d1; ++d) dot += qs[g * hd + d] * static_cast<float>(krow[d]);
-                dot = lanes_sum<4>(dot);
-                if (valid && sub == 0) sc[g * kPAttnChunk + tt] = dot * rscale;
-            }
-        }
-        __syncthreads();
-        // online softmax update per head (one wave per head)
-        for (int g = wid; g < group; g += blockDim.x / kWave) {
-            const float sv = lane < n ? sc[g * kPAttnChunk + lane] : -INFINITY;
-            const float mc = wave_max(sv);
-            const float m_old = ml[2 * g];
-            const float m_new = fmaxf(m_old, mc);
-            const float e = lane < n ? expf(sv - m_new) : 0.0f;
-            const float lsum = wave_sum(e);
-            sc[g * kPAttnChunk + lane] = e;
-            if (lane == 0) {
-                const float f = expf(m_old - m_new);  // 0 for the first chunk
-                fac[g] = f;
-                ml[2 * g] = m_new;
-                ml[2 * g + 1] = ml[2 * g + 1] * f + lsum;
-            }
-        }
-        __syncthreads();
-        for (int i = threadIdx.x; i < group * hd; i += blockDim.x) {
-            const int g = i / hd, d = i % hd;
-            float o = osum[i] * fac[g];
-            for (int j = 0; j < n; ++j)
-                o += sc[g * kPAttnChunk + j] *
-                     static_cast<float>(p.v_cache[(static_cast<size_t>(c0 + j) * p.nkv + kh) * hd + d]);
-            osum[i] = o;
-        }
-        __syncthreads();
-    }
-    for (int i = threadIdx.x; i < group * hd; i += blockDim.x) {
-        const int g = i / hd;
-        const float l = ml[2 * g + 1];
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        const size_t oi = static_cast<size_t>(t) * p.out_stride + static_cast<size_t>(kh) * group * hd + i;
-        const size_t gi = static_cast<size_t>(t) * p.q_stride + static_cast<size_t>(kh) * group * hd + i;
-        p.out[oi] = (osum[i] * inv) * sigmoid_dev(p.gate[gi]);
-    }
-}
-
-// Matrix-core form for head_dim 128 and 4 query heads per kv head (the 9B
-// shape): block (16-token tile, kv head), wave h = query head h of the kv head,
-// keys in 64-key chunks with a running max / sum (rescaled by
-// exp(m_old - m_new)), then 1/l and the sigmoid gate, as prefill_attn_kernel.
-// Scores are formed transposed, S^T = K Q^T (keys are the MFMA rows), so a
-// lane holds 16 keys of one token: the token's max and sum are over the lane's
-// own values and the lanes 16 and 32 away, and its probabilities are already
-// the B operand of O^T = V^T P^T.  q and p are split into fp16 hi + lo (about
-// 22 bits together; k and v are fp16 in the cache), two
-// v_mfma_f32_16x16x32_f16 per product, fp32 accumulation.  The k index of an
-// MFMA may be any permutation of the keys as long as both operands use it:
-// lane group g (lanes 16g..16g+15) feeds keys 32s + 4g + 0..3 and
-// 32s + 16 + 4g + 0..3 of step s, the keys its score tiles hold.  A chunk's K
-// (rows of 128 dims) and V (transposed: rows of 64 keys) go through LDS; the
-// next chunk is loaded into registers while the current one is used.
-constexpr int kFT = 16;        // tokens per tile
-constexpr int kFLdk = 136;     // halves per K row in LDS
-constexpr int kFLdv = 72;      // halves per V^T row in LDS
-constexpr int kFHd = 128, kFGroup = 4;
-
-template <int M>
-__device__ __forceinline__ float xor_pair_max(float v) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, v);
-    if constexpr (M == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-        return fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(r[0])),
-                     __builtin_bit_cast(float, static_cast<uint32_t>(r[1])));
-    } else {
-        static_assert(M == 32, "pair distance");
-        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-        return fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(r[0])),
-                     __builtin_bit_cast(float, static_cast<uint32_t>(r[1])));
-    }
-}
-
-// fp32 -> fp16 hi + fp16 lo (x - hi) of 8 values
-__device__ __forceinline__ void split_h8(const float (&x)[8], half8& hi, half8& lo) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const _Float16 h = static_cast<_Float16>(x[e]);
-        hi[e] = h;
-        lo[e] = static_cast<_Float16>(x[e] - static_cast<float>(h));
-    }
-}
-
-__global__ void __launch_bounds__(256) prefill_attn_mfma_kernel(PrefillAttnLaunch p) {
-    __shared__ _Float16 Ks[kPAttnChunk * kFLdk];
-    __shared__ _Float16 Vt[kFHd * kFLdv];
-    const int t0 = blockIdx.x * kFT, kh = blockIdx.y;
-    const int lane = threadIdx.x & (kWave - 1), h = threadIdx.x / kWave;
-    const int tl = lane & 15, g = lane >> 4;
-    // block-uniform values computed with vector ops are made scalar with
-    // readfirstlane: a buffer descriptor built from a vector register becomes a
-    // loop over the distinct values of the wave
-    const int pos0 = *p.pos0;
-    const int ntok = __builtin_amdgcn_readfirstlane(min(kFT, p.tokens - t0));
-    const int qpos = pos0 + t0 + tl;        // this lane's token
-    const int last = pos0 + t0 + ntok - 1;  // last key any token of the tile sees
-    const int qh = kh * kFGroup + h;
-    const float rscale = 1.0f / sqrtf(static_cast<float>(kFHd));
-    // q fragments: lane supplies Q[token tl][dims 32 s + 8 g .. + 7] (tokens past ntok read 0)
-    const uint32_t qrow = static_cast<uint32_t>(p.q_stride) * 4u;
-    const __amdgpu_buffer_rsrc_t r_q = buf_rsrc(p.q + static_cast<size_t>(t0) * p.q_stride, ntok * qrow);
-    half8 qhi[4], qlo[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const uint32_t off = static_cast<uint32_t>(tl) * qrow + (static_cast<uint32_t>(qh) * kFHd + 32 * s + 8 * g) * 4u;
-        const auto a = __builtin_amdgcn_raw_buffer_load_b128(r_q, off, 0, 0);
-        const auto b = __builtin_amdgcn_raw_buffer_load_b128(r_q, off + 16u, 0, 0);
-        const float x[8] = {__uint_as_float(a[0]), __uint_as_float(a[1]), __uint_as_float(a[2]), __uint_as_float(a[3]),
-                            __uint_as_float(b[0]), __uint_as_float(b[1]), __uint_as_float(b[2]), __uint_as_float(b[3])};
-        split_h8(x, qhi[s], qlo[s]);
-    }
-    // chunk loads: piece i = threadIdx + 256 u is key i & 63, dims 8 (i >> 6) .. + 7
-    const uint32_t krow = static_cast<uint32_t>(p.nkv) * kFHd * 2u;  // bytes per cache position
-    u32x4 kr[4], vr[4];
-    auto load_chunk = [&](int c0) {
-        const uint32_t range =
-            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(max(0, min(kPAttnChunk, last - c0 + 1)))) * krow;
-        const size_t base = static_cast<size_t>(__builtin_amdgcn_readfirstlane(max(0, min(c0, last)))) * p.nkv * kFHd +
-                            static_cast<size_t>(kh) * kFHd;
-        const __amdgpu_buffer_rsrc_t rk = buf_rsrc(p.k_cache + base, range), rv = buf_rsrc(p.v_cache + base, range);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = static_cast<int>(threadIdx.x) + 256 * u;
-            const uint32_t off = static_cast<uint32_t>(i & 63) * krow + static_cast<uint32_t>(i >> 6) * 16u;
-            kr[u] = __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0);
-            vr[u] = __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0);
-        }
-    };
-    float m = -INFINITY, l = 0.0f;
-    floatx4 o[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    load_chunk(0);
-    for (int c0 = 0; c0 <= last; c0 += kPAttnChunk) {  // block-uniform
-        __syncthreads();  // the previous chunk's K and V have been read
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = static_cast<int>(threadIdx.x) + 256 * u, key = i & 63, d8 = i >> 6;
-            *reinterpret_cast<u32x4*>(Ks + key * kFLdk + 8 * d8) = kr[u];
-            const uint32_t w[4] = {vr[u][0], vr[u][1], vr[u][2], vr[u][3]};
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                Vt[(8 * d8 + e) * kFLdv + key] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1))));
-        }
-        __syncthreads();
-        load_chunk(c0 + kPAttnChunk);  // past `last`: reads 0, never stored as data
-        // S^T tiles c: keys c0 + 16 c + 4 g + v of token tl
-        floatx4 sc[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sc[c] = zero4;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const half8 a = *reinterpret_cast<const half8*>(Ks + (16 * c + tl) * kFLdk + 32 * s + 8 * g);
-                sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qhi[s], sc[c], 0, 0, 0);
-                sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qlo[s], sc[c], 0, 0, 0);
-            }
-        }
-        // causal mask, the token's chunk max and sum, online rescale
-        float mc = -INFINITY;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const bool ok = c0 + 16 * c + 4 * g + v <= qpos;
-                sc[c][v] = ok ? sc[c][v] * rscale : -INFINITY;
-                mc = fmaxf(mc, sc[c][v]);
-            }
-        mc = xor_pair_max<32>(xor_pair_max<16>(mc));
-        const float m_new = fmaxf(m, mc);
-        float ls = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float e = sc[c][v] == -INFINITY ? 0.0f : expf(sc[c][v] - m_new);
-                sc[c][v] = e;
-                ls += e;
-            }
-        ls = xor_pair_sum<32>(xor_pair_sum<16>(ls));
-        const float f = m == -INFINITY ? 0.0f : expf(m - m_new);
-        m = m_new;
-        l = l * f + ls;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] *= f;
-        // P^T fragments of key steps s2 (keys 32 s2 + 4 g + v, then 32 s2 + 16 + 4 g + v)
-        half8 phi[2], plo[2];
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            const float x[8] = {sc[2 * s2][0], sc[2 * s2][1], sc[2 * s2][2], sc[2 * s2][3],
-                                sc[2 * s2 + 1][0], sc[2 * s2 + 1][1], sc[2 * s2 + 1][2], sc[2 * s2 + 1][3]};
-            split_h8(x, phi[s2], plo[s2]);
-        }
-        // O^T tiles j: dims 16 j + 4 g + v of token tl
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                const _Float16* vrow = Vt + (16 * j + tl) * kFLdv + 32 * s2 + 4 * g;
-                const u32x2 lo4 = *reinterpret_cast<const u32x2*>(vrow);
-                const u32x2 hi4 = *reinterpret_cast<const u32x2*>(vrow + 16);
-                const half8 a = __builtin_bit_cast(half8, u32x4{lo4[0], lo4[1], hi4[0], hi4[1]});
-                o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, phi[s2], o[j], 0, 0, 0);
-                o[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, plo[s2], o[j], 0, 0, 0);
-            }
-    }
-    if (tl >= ntok) return;
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const size_t head = static_cast<size_t>(qh) * kFHd + 4 * g;
-    const float* gr = p.gate + static_cast<size_t>(t0 + tl) * p.q_stride + head;
-    float* orow = p.out + static_cast<size_t>(t0 + tl) * p.out_stride + head;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float4 gv = *reinterpret_cast<const float4*>(gr + 16 * j);
-        *reinterpret_cast<float4*>(orow + 16 * j) =
-            make_float4((o[j][0] * inv) * sigmoid_dev(gv.x), (o[j][1] * inv) * sigmoid_dev(gv.y),
-                        (o[j][2] * inv) * sigmoid_dev(gv.z), (o[j][3] * inv) * sigmoid_dev(gv.w));
-    }
-}
-
-bool prefill_attn_supported(int nq, int nkv, int head_dim) {
-    return nkv > 0 && nq % nkv == 0 && nq / nkv <= kPAttnMaxGroup && head_dim > 0 &&
-           sizeof(float) * (2 * (nq / nkv) * head_dim + (nq / nkv) * (kPAttnChunk + 3)) <= 64 * 1024;
-}
-
-hipError_t launch_prefill_attn(const PrefillAttnLaunch& p, hipStream_t s) {
-    const int group = p.nq / p.nkv;
-    // the matrix-core kernel reads q, the gate and the output as 16-byte pieces
-    const bool al16 = ((reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.gate) |
-                        reinterpret_cast<uintptr_t>(p.out)) & 15u) == 0 && p.q_stride % 4 == 0 && p.out_stride % 4 == 0;
-    if (p.head_dim == kFHd && group == kFGroup && al16) {
-        hipLaunchKernelGGL(prefill_attn_mfma_kernel, dim3((p.tokens + kFT - 1) / kFT, p.nkv), dim3(256), 0, s, p);
-        return hipGetLastError();
-    }
-    const size_t lds = sizeof(float) * (2 * static_cast<size_t>(group) * p.head_dim + group * (kPAttnChunk + 3));
-    hipLaunchKernelGGL(prefill_attn_kernel, dim3(p.tokens, p.nkv), dim3(256), lds, s, p);
     return hipGetLastError();
 }
 
