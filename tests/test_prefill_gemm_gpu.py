@@ -1,0 +1,71 @@
+"""The prefill GEMM's three tiles and its K splits against the dequantised
+product in 64 bits (gemvW4A16Neon per token, xq_gemv_w4a16_neon.cpp:259-291), at
+sizes that leave each tile, quad of groups and split partly empty, in the four
+metadata forms.
+
+Bound: x carries 22 bits (fp16 hi + lo: 2^-22 of itself), the codes are exact, the
+zero-point term's factors carry 22 bits each, and the fp32 sums round once per
+MFMA and group: |error| <= (2^-20 + (8 G + 16) 2^-24 / 4) sum |w| |x|, the last
+term with its roundings' signs averaging out to a quarter of their worst case."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import xqbind as xb
+from test_decode_ops_gpu import dev
+
+pytestmark = pytest.mark.gpu
+
+
+def matrix(rng, rows, cols, form):
+    """(packed, scales, zeros, affine, dense fp64) in the metadata form: `s16` fp16 scale and zero 8, `f16` fp16
+    pairs, `z4` fp32 scale and integer zero, `f32` fp32 pairs (affine)."""
+    n = rows * cols // 64
+    packed = rng.integers(0, 256, rows * cols // 2, dtype=np.uint8)
+    scales = np.abs(rng.normal(0, 0.02, n)).astype(np.float32)
+    if form in ("s16", "f16"):
+        scales = scales.astype(np.float16).astype(np.float32)
+    zeros = {"s16": np.full(n, 8.0), "f16": np.round(rng.normal(0, 4, n)) / 8, "z4": rng.integers(0, 16, n).astype(float),
+             "f32": rng.normal(0, 0.1, n)}[form].astype(np.float32)
+    affine = 1 if form in ("f16", "f32") else 0
+    q = np.stack([packed & 15, packed >> 4], -1).reshape(rows, cols // 64, 64).astype(np.float64)
+    s, z = scales.astype(np.float64).reshape(rows, -1, 1), zeros.astype(np.float64).reshape(rows, -1, 1)
+    return packed, scales, zeros, affine, (q * s + z if affine else (q - z) * s).reshape(rows, cols)
+
+
+@pytest.mark.parametrize("form", ["s16", "f16", "z4", "f32"])
+@pytest.mark.parametrize("rows,cols,m,epi", [
+    (128, 512, 1, "store"), (129, 1024, 32, "add"), (34, 4160, 33, "silu"), (1000, 640, 31, "store"),  # small tile
+    (258, 2048, 7, "silu"), (96, 12288, 40, "add"),                                                    # ... split
+    (20001, 576, 130, "add"), (20000, 64, 129, "silu"), (24600, 320, 500, "store"),                     # middle tile
+    (20002, 192, 257, "store"), (19970, 448, 300, "add"), (20000, 256, 384, "silu")])                   # large tile
+def test_matches_64_bit_product(rows, cols, m, epi, form):
+    rng = np.random.default_rng(rows + cols + m)
+    packed, scales, zeros, affine, W = matrix(rng, rows, cols, form)
+    w = xb.DeviceW4(packed, scales, zeros, rows, cols, affine=affine)
+    ldx, out = cols + 4, rows // 2 if epi == "silu" else rows
+    ldy = out + 3
+    x = rng.normal(0, 1, (m, ldx)).astype(np.float32)
+    y0 = rng.normal(0, 1, (m, ldy)).astype(np.float32)
+    yd = dev(y0)
+    ws = xb.DeviceBuffer(xb.hip().xqhip_gemm_workspace_bytes(m, cols, rows))
+    code = {"store": xb.EPI_STORE, "add": xb.EPI_ADD, "silu": xb.EPI_SILU_PAIR}[epi]
+    xb.ck(xb.hip().xqhip_gemm_w4a16(w.ref, dev(x).ptr, m, ldx, None, 0, yd.ptr, ldy, code, ws.ptr, ws.nbytes, None))
+    got = yd.download(np.float32, m * ldy).reshape(m, ldy)
+    assert np.array_equal(got[:, out:], y0[:, out:])
+    x64 = x[:, :cols].astype(np.float64)
+    y, size = x64 @ W.T, np.abs(x64) @ np.abs(W).T
+    G = cols // 64
+    tol = (2.0**-20 + (8 * G + 16) * 2.0**-26) * size + 1e-7
+    if epi == "silu":
+        g, u = y[:, 0::2], y[:, 1::2]
+        sig = 1 / (1 + np.exp(-g))
+        # |silu'| <= 1.1; expf and the divide: 4 ulp
+        tol = 1.1 * np.abs(u) * tol[:, 0::2] + (np.abs(g * sig) + tol[:, 0::2]) * tol[:, 1::2] + 2.0**-21 * np.abs(g * sig * u)
+        y = g * sig * u
+    elif epi == "add":
+        y = y0[:, :out] + y
+        tol = tol + 2.0**-23 * np.abs(y)
+    err = np.abs(got[:, :out] - y)
+    assert (err <= tol).all(), (err / tol).max()

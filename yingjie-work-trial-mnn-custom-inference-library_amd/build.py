@@ -49,7 +49,7 @@ HIP_FLAGS = [
 ]
 # per-source additions: the prefill GEMM scales every MFMA result with VALU ops, so its
 # MFMAs write VGPRs directly instead of accumulation registers that need copying out
-HIP_FILE_FLAGS = {"prefill_ops.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+HIP_FILE_FLAGS = {"prefill_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter",
               "-fvisibility=hidden", "-I", INCLUDE, "-I", HOST_SRC, "-DXQWEN35_BUILD=1"]
 

@@ -1,17 +1,10 @@
-// prefill_ops.hip - the multi-token (prefill) kernels of the decode path on gfx950.
+// prefill_ops.hip - linear attention of a prompt chunk on gfx950.
 //
 // The reference prefills token by token (CustomModel::prefill,
 // customlib/runtime/custom_model.cpp:610-640); the arithmetic per token is the
-// same as decode.  Here the dense contractions of a prompt chunk (the
-// q/k/v/o, gate/up and down projections of every layer for up to
-// kPrefillChunk tokens) run as one W4A16 GEMM each on the matrix cores, and
-// the sequential parts run as batched kernels:
-//   prep_x_kernel        per-token RMSNorm / gated head norm, x -> fp16 hi + lo
-//                        and per-group sums of x
-//   gemm_w4_mfma_kernel  per 64-column group: codes q - 8 (exact in fp16) times
-//                        x hi / lo on v_mfma_f32_16x16x32_f16, group sums scaled
-//                        by the group scale; the zero-point term as a K = G
-//                        MFMA contraction after the group loop
+// same as decode.  The chunk's projections are in prefill_gemm.hip, its
+// attention in prefill_attn.hip; here the recurrence of the linear-attention
+// layers runs as batched kernels:
 //   linear_conv_prefill_tg_kernel + scan_chunk_prep_kernel + scan_chunk_state_kernel   conv1d + norms +
 //                        gates for all tokens, then the gated-delta recurrence
 //                        with the state in registers (one-pass kernels
@@ -23,726 +16,9 @@
 
 namespace xqhip {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 // register arrays of native vectors (arrays of HIP's uint4 / uint2 structs are kept in scratch)
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack_h2(_Float16 lo, _Float16 hi) {
-    return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, lo)) |
-           (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, hi)) << 16);
-}
-
-// ---------------------------------------------------------------------------
-// B operand preparation: token t = blockIdx.x of x (row stride ldx) with the
-// prologue applied (RMS over the row, or per-head gated norm with the gate
-// row at t * ldz) -> v, stored as xh = fp16(v) and xl = fp16(v - xh) (about
-// 22 significant bits together) with every aligned run of 8 columns in the
-// order [0 4 1 5 2 6 3 7], the order in which the GEMM unpacks a word of 8
-// weight codes; xs[t][g] = fp32 sum of v over column group g (64 columns).
-// Each row is first scaled by a power of two, ts[t] = 2^k, that brings its
-// largest magnitude into [2^12, 2^13): fp16 then holds any fp32 activation
-// (silu(gate) * up of a large residual stream can exceed 65504) without
-// overflow or subnormal loss, and the GEMM multiplies its results by ts[t]
-// (exact).  Rows m..m_pad-1 are zero-filled (ts 1).
-// ---------------------------------------------------------------------------
-constexpr int kPrepMaxHeads = 256;
-
-__global__ void __launch_bounds__(256) prep_x_kernel(const float* __restrict__ x, int ldx, int m, int cols,
-                                                     Prologue pro, int ldz, _Float16* __restrict__ xh,
-                                                     _Float16* __restrict__ xl, float* __restrict__ xs,
-                                                     float* __restrict__ ts) {
-    __shared__ float red[32];
-    __shared__ float head_inv[kPrepMaxHeads];
-    const int t = blockIdx.x;
-    const int G = cols >> 6, nch = cols >> 3;
-    uint4* oh = reinterpret_cast<uint4*>(xh + static_cast<size_t>(t) * cols);
-    uint4* ol = reinterpret_cast<uint4*>(xl + static_cast<size_t>(t) * cols);
-    float* os = xs + static_cast<size_t>(t) * G;
-    if (t >= m) {
-        for (int c = threadIdx.x; c < nch; c += blockDim.x) oh[c] = ol[c] = make_uint4(0u, 0u, 0u, 0u);
-        for (int g = threadIdx.x; g < G; g += blockDim.x) os[g] = 0.0f;
-        if (threadIdx.x == 0) ts[t] = 1.0f;
-        return;
-    }
-    const float* xr = x + static_cast<size_t>(t) * ldx;
-    const float* zr = pro.mode == PRO_GATED ? pro.z + static_cast<size_t>(t) * ldz : nullptr;
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave, nw = blockDim.x / kWave;
-    float inv = 1.0f;
-    if (pro.mode == PRO_RMS) {
-        float ss = 0.0f;
-        for (int c = threadIdx.x; c < cols; c += blockDim.x) ss += xr[c] * xr[c];
-        ss = block_sum(ss, red);
-        inv = 1.0f / sqrtf(ss / static_cast<float>(cols) + pro.eps);
-    } else if (pro.mode == PRO_GATED) {
-        const int heads = cols / pro.head_dim;
-        for (int h = wid; h < heads; h += nw) {  // one wave per head
-            const float* xv = xr + h * pro.head_dim;
-            float ss = 0.0f;
-            for (int d = lane; d < pro.head_dim; d += kWave) ss += xv[d] * xv[d];
-            ss = wave_sum(ss);
-            if (lane == 0) head_inv[h] = 1.0f / sqrtf(ss / static_cast<float>(pro.head_dim) + pro.eps);
-        }
-        __syncthreads();
-    }
-    // one thread per 8 columns; the 8 threads of a group are consecutive lanes (nch % 8 == 0)
-    auto load8 = [&](int c, float (&v)[8]) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = xr[c + e];
-        if (pro.mode == PRO_RMS) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = v[e] * inv * pro.w[c + e];
-        } else if (pro.mode == PRO_GATED) {
-            const int h = c / pro.head_dim, d = c - h * pro.head_dim;  // head_dim % 8 == 0
-            const float ih = head_inv[h];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = v[e] * ih * pro.w[d + e] * silu_dev(zr[c + e]);
-        }
-    };
-    // the row's power-of-two scale from its largest magnitude
-    float mx = 0.0f;
-    for (int c8 = threadIdx.x; c8 < nch; c8 += blockDim.x) {
-        float v[8];
-        load8(c8 * 8, v);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[e]));
-    }
-    mx = wave_max(mx);
-    __syncthreads();  // red may still be read by the norm's block_sum
-    if (lane == 0) red[wid] = mx;
-    __syncthreads();
-    for (int i = 0; i < nw; ++i) mx = fmaxf(mx, red[i]);
-    int ex = 0;
-    frexpf(mx, &ex);                                       // mx = f 2^ex, f in [0.5, 1)
-    const float down = mx > 0.0f ? ldexpf(1.0f, 13 - ex) : 1.0f;  // mx * down in [2^12, 2^13)
-    if (threadIdx.x == 0) ts[t] = mx > 0.0f ? ldexpf(1.0f, ex - 13) : 1.0f;
-    for (int c8 = threadIdx.x; c8 < nch; c8 += blockDim.x) {
-        const int c = c8 * 8;
-        float v[8];
-        load8(c, v);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= down;
-        uint32_t ph[4], pl[4];
-        float sum = 0.0f;
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {  // positions 2p, 2p + 1 <- columns p, p + 4
-            const float va = v[p], vb = v[p + 4];
-            const _Float16 ha = static_cast<_Float16>(va), hb = static_cast<_Float16>(vb);
-            ph[p] = pack_h2(ha, hb);
-            pl[p] = pack_h2(static_cast<_Float16>(va - static_cast<float>(ha)),
-                            static_cast<_Float16>(vb - static_cast<float>(hb)));
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sum += v[e];
-        oh[c8] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-        ol[c8] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-        sum = lanes_sum<8>(sum);
-        if ((c8 & 7) == 0) os[c8 >> 3] = sum;
-    }
-}
-
-// The same for rows of NK * 2048 columns with 16-byte aligned rows, weights and
-// gates, the prologue mode a template argument: thread i owns the 8-column
-// pieces i, i + 256, ... of its token's row and loads each once, as 16-byte
-// loads with no branch around them (the generic kernel reads the row three
-// times, one float per load); the gated norm's per-head sums stay inside the
-// 16 lanes that own a 128-column head.
-template <int NK, int MODE>
-__global__ void __launch_bounds__(256) prep_x_vec_kernel(const float* __restrict__ x, int ldx, int m, Prologue pro,
-                                                         int ldz, _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                         float* __restrict__ xs, float* __restrict__ ts) {
-    constexpr int kCols = NK * 2048, kG = kCols / 64;
-    __shared__ float red_s[4], red_m[4];
-    const int t = blockIdx.x;
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    uint4* oh = reinterpret_cast<uint4*>(xh + static_cast<size_t>(t) * kCols);
-    uint4* ol = reinterpret_cast<uint4*>(xl + static_cast<size_t>(t) * kCols);
-    float* os = xs + static_cast<size_t>(t) * kG;
-    if (t >= m) {  // block-uniform
-#pragma unroll
-        for (int k = 0; k < NK; ++k) oh[threadIdx.x + 256 * k] = ol[threadIdx.x + 256 * k] = make_uint4(0u, 0u, 0u, 0u);
-        for (int g = threadIdx.x; g < kG; g += 256) os[g] = 0.0f;
-        if (threadIdx.x == 0) ts[t] = 1.0f;
-        return;
-    }
-    const float4* xr = reinterpret_cast<const float4*>(x + static_cast<size_t>(t) * ldx);
-    float4 xv[NK][2], wv[NK][2], zv[NK][2];
-#pragma unroll
-    for (int k = 0; k < NK; ++k) {
-        const int c4 = 2 * (threadIdx.x + 256 * k);  // float4 index of the piece
-        xv[k][0] = xr[c4];
-        xv[k][1] = xr[c4 + 1];
-        if constexpr (MODE == PRO_RMS) {
-            wv[k][0] = reinterpret_cast<const float4*>(pro.w)[c4];
-            wv[k][1] = reinterpret_cast<const float4*>(pro.w)[c4 + 1];
-        } else if constexpr (MODE == PRO_GATED) {
-            // head_dim 128: the piece's offset in its head is 8 (i mod 16)
-            const int d4 = 2 * (threadIdx.x & 15);
-            wv[k][0] = reinterpret_cast<const float4*>(pro.w)[d4];
-            wv[k][1] = reinterpret_cast<const float4*>(pro.w)[d4 + 1];
-            const float4* zr = reinterpret_cast<const float4*>(pro.z + static_cast<size_t>(t) * ldz);
-            zv[k][0] = zr[c4];
-            zv[k][1] = zr[c4 + 1];
-        }
-    }
-    float v[NK][8];
-#pragma unroll
-    for (int k = 0; k < NK; ++k) {
-        const float4 a = xv[k][0], b = xv[k][1];
-        v[k][0] = a.x; v[k][1] = a.y; v[k][2] = a.z; v[k][3] = a.w;
-        v[k][4] = b.x; v[k][5] = b.y; v[k][6] = b.z; v[k][7] = b.w;
-    }
-    if constexpr (MODE == PRO_RMS) {
-        float ss = 0.0f;
-#pragma unroll
-        for (int k = 0; k < NK; ++k)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ss += v[k][e] * v[k][e];
-        ss = wave_sum(ss);
-        if (lane == 0) red_s[wid] = ss;
-        __syncthreads();
-        ss = (red_s[0] + red_s[1]) + (red_s[2] + red_s[3]);
-        const float inv = 1.0f / sqrtf(ss / static_cast<float>(kCols) + pro.eps);
-#pragma unroll
-        for (int k = 0; k < NK; ++k) {
-            const float w8[8] = {wv[k][0].x, wv[k][0].y, wv[k][0].z, wv[k][0].w,
-                                 wv[k][1].x, wv[k][1].y, wv[k][1].z, wv[k][1].w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[k][e] = v[k][e] * inv * w8[e];
-        }
-    } else if constexpr (MODE == PRO_GATED) {
-#pragma unroll
-        for (int k = 0; k < NK; ++k) {
-            float ss = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ss += v[k][e] * v[k][e];
-            ss = lanes_sum<16>(ss);  // the head's 16 pieces
-            const float ih = 1.0f / sqrtf(ss / 128.0f + pro.eps);
-            const float w8[8] = {wv[k][0].x, wv[k][0].y, wv[k][0].z, wv[k][0].w,
-                                 wv[k][1].x, wv[k][1].y, wv[k][1].z, wv[k][1].w};
-            const float z8[8] = {zv[k][0].x, zv[k][0].y, zv[k][0].z, zv[k][0].w,
-                                 zv[k][1].x, zv[k][1].y, zv[k][1].z, zv[k][1].w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[k][e] = v[k][e] * ih * w8[e] * silu_dev(z8[e]);
-        }
-    }
-    // the row's power-of-two scale from its largest magnitude
-    float mx = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NK; ++k)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[k][e]));
-    mx = wave_max(mx);
-    if (lane == 0) red_m[wid] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
-    int ex = 0;
-    frexpf(mx, &ex);
-    const float down = mx > 0.0f ? ldexpf(1.0f, 13 - ex) : 1.0f;
-    if (threadIdx.x == 0) ts[t] = mx > 0.0f ? ldexpf(1.0f, ex - 13) : 1.0f;
-#pragma unroll
-    for (int k = 0; k < NK; ++k) {
-        const int c8 = threadIdx.x + 256 * k;
-        uint32_t ph[4], pl[4];
-        float sum = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[k][e] *= down;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {  // positions 2q, 2q + 1 <- columns q, q + 4
-            const float va = v[k][q], vb = v[k][q + 4];
-            const _Float16 ha = static_cast<_Float16>(va), hb = static_cast<_Float16>(vb);
-            ph[q] = pack_h2(ha, hb);
-            pl[q] = pack_h2(static_cast<_Float16>(va - static_cast<float>(ha)),
-                            static_cast<_Float16>(vb - static_cast<float>(hb)));
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sum += v[k][e];
-        oh[c8] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-        ol[c8] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-        sum = lanes_sum<8>(sum);
-        if ((c8 & 7) == 0) os[c8 >> 3] = sum;
-    }
-}
-
-// the vectorised form's launch, or false when the shape or alignment needs the generic kernel
-template <int NK>
-static bool launch_prep_vec(const GemmLaunch& p, int m_pad, _Float16* xh, _Float16* xl, float* xs, float* ts,
-                            hipStream_t s) {
-    if (p.pro.mode == PRO_RMS)
-        hipLaunchKernelGGL((prep_x_vec_kernel<NK, PRO_RMS>), dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.pro,
-                           p.ldz, xh, xl, xs, ts);
-    else if (p.pro.mode == PRO_GATED)
-        hipLaunchKernelGGL((prep_x_vec_kernel<NK, PRO_GATED>), dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.pro,
-                           p.ldz, xh, xl, xs, ts);
-    else
-        hipLaunchKernelGGL((prep_x_vec_kernel<NK, PRO_NONE>), dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.pro,
-                           p.ldz, xh, xl, xs, ts);
-    return true;
-}
-
-static bool prep_vec_ok(const GemmLaunch& p) {
-    auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
-    if (p.cols % 2048 != 0 || !al16(p.x) || p.ldx % 4 != 0) return false;
-    if (p.pro.mode == PRO_RMS) return al16(p.pro.w);
-    if (p.pro.mode == PRO_GATED) return p.pro.head_dim == 128 && al16(p.pro.w) && al16(p.pro.z) && p.ldz % 4 == 0;
-    return p.pro.mode == PRO_NONE;
-}
-
-// ---------------------------------------------------------------------------
-// W4A16 GEMM, y[t][r] (op)= sum_k w[r][k] x[t][k] for a prompt chunk.
-//
-// In column group g (64 columns) a row's weights are w = sn s + c0 with
-// sn = q - 8 the signed code, s the group scale and c0 = (8 - z) s for
-// w = (q - z) s, or 8 s + z for w = q s + z.  Hence
-//     y[t][r] = sum_g s[r][g] A[r][t][g] + sum_g c0[r][g] xs[t][g],
-//     A[r][t][g] = sum_{k in g} sn[r][k] x[t][k],  xs[t][g] = sum_{k in g} x[t][k].
-// sn is exact in fp16, so A takes two v_mfma_f32_16x16x32_f16 passes per 32
-// columns (sn x_hi + sn x_lo, x = x_hi + x_lo to about 22 bits) into a
-// per-group accumulator, which is scaled by s into the fp32 result.  The c0
-// term is a K = G contraction done after the group loop in three fp16 hi/lo
-// passes (c0 scaled by 64 and xs by 1/64, both exact, to stay in fp16 range).
-//
-// Block: WGR x WGT waves, each owning TI x TJ tiles of 16 rows x 16 tokens.
-// A operand: each lane loads its 8 bytes of a tile row's group straight from
-// the TILED64 matrix into registers, in a four-group ring ahead of the MFMAs:
-// lane l takes row l & 15 and words 2 (q & 1), 2 (q & 1) + 1 of half q >> 1,
-// q = l >> 4 (columns 32 (q >> 1) + 16 (q & 1) + 0..15), and unpacks a word
-// of 8 codes to fp16 q - 8 with integer ops ((u >> 4j) & 0x000F000F | 0x64006400
-// is fp16 1024 + q for codes j and j + 4) and one packed fp16 subtraction.
-// B operand: the block's BT tokens x 64 columns of x_hi and x_lo go through a
-// register ring two groups ahead into double-buffered LDS, one barrier per
-// group, with the scales of the block's rows.
-// MFMA operand layout (16x16x32): lane l supplies row/column (l & 15) and 8
-// consecutive k at 8 (l >> 4); lane l receives D[4 (l >> 4) + v][l & 15].
-// Here the k of an MFMA is a permutation of the group's columns, the same for
-// both operands.  Token tiles are the fastest grid dimension, so the blocks
-// that share a weight tile run together and it is fetched from HBM about once.
-// ---------------------------------------------------------------------------
-constexpr int kGemmPad = 128;  // xh / xl / xs rows are padded to a multiple of this
-
-struct GemmArgs {
-    const uint8_t* nib;
-    const uint32_t* meta;
-    int rows, cols, affine;
-    int zero_is_8;       // c0 = (8 - z) s is 0 for every group: the c0 pass is skipped
-    const _Float16* xh;  // [m_pad][cols], followed by xl [m_pad][cols]
-    const float* xs;     // [m_pad][cols / 64]
-    const float* ts;     // [m_pad] per-token power-of-two scale of xh / xl / xs
-    int gps;             // column groups per K split (blockIdx.z); the whole row when unsplit
-    float* part;         // split K: [gridDim.z][m][rows] partial products (the reduce applies EPI)
-    int m, m_pad;
-    float* y;
-    int ldy;
-};
-
-constexpr int kGemmXLd = 136;  // LDS x row in halves: x_hi[64] | x_lo[64] | 8 padding
-
-template <int WGR, int WGT, int TI, int TJ>
-struct GemmTile {
-    static constexpr int kWaves = WGR * WGT, kThreads = kWave * kWaves;
-    static constexpr int kWR = 16 * TI, kWT = 16 * TJ, kBR = WGR * kWR, kBT = WGT * kWT;
-    static constexpr int kXU = kBT * 16 / kThreads;  // 16-byte pieces of x per thread per group
-    static constexpr int kXStage = kBT * kGemmXLd;   // halves per stage
-    static constexpr size_t kLds = 2 * (static_cast<size_t>(kXStage) * sizeof(_Float16) + kBR * sizeof(float));
-    static_assert(kXU * kThreads == kBT * 16, "x staging");
-    static_assert(kBR <= kThreads, "scale staging");
-};
-
-// 8 stored codes (q ^ 8; column n of the word in bits 4n..4n+3) -> fp16 q - 8
-// in the column order [0 4 1 5 2 6 3 7]: ((w >> 4j) & 0x000F000F) ^ 0x64086408
-// is fp16 (1024 + q) for the codes j and j + 4 (one shift and one three-input
-// bit op), less 1032 in one packed fp16 subtraction.
-__device__ __forceinline__ half8 codes_to_h8(uint32_t w) {
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    const half2_t bias = {static_cast<_Float16>(1032.0f), static_cast<_Float16>(1032.0f)};
-    uint32_t p[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const half2_t h = __builtin_bit_cast(half2_t, ((w >> (4 * j)) & 0x000F000Fu) ^ 0x64086408u) - bias;
-        p[j] = __builtin_bit_cast(uint32_t, h);
-    }
-    return __builtin_bit_cast(half8, make_uint4(p[0], p[1], p[2], p[3]));
-}
-
-// two waves per SIMD (at most 256 registers per lane), so one block's barrier wait overlaps another's work
-template <int WGR, int WGT, int TI, int TJ, int EPI, int META>
-__global__ void __launch_bounds__(kWave * WGR * WGT) __attribute__((amdgpu_waves_per_eu(2)))
-gemm_w4_mfma_kernel(GemmArgs a) {
-    // fp16 (scale, zero) in a u32, the fp32 pair (the scale is its first word), the fp16 scale alone,
-    // or the fp32 scale (its zero in the separate array of 4-bit codes)
-    constexpr uint32_t kMetaBytes = kMetaGroupBytes<META>;
-    using T = GemmTile<WGR, WGT, TI, TJ>;
-    constexpr int BR = T::kBR, BT = T::kBT, XU = T::kXU, NT = T::kThreads;
-    constexpr int kTokStep = NT / 16;  // tokens between a thread's x pieces
-    extern __shared__ uint4 gemm_lds[];
-    _Float16* xlds = reinterpret_cast<_Float16*>(gemm_lds);         // [2 stages][BT][kGemmXLd]
-    float* slds = reinterpret_cast<float*>(xlds + 2 * T::kXStage);  // [2 stages][BR] scales
-    // Tile of this block.  Blocks are dealt to the 8 XCDs round robin in
-    // launch order; a weight slab (128 rows of one K split, a "unit") is read
-    // by every token tile, so the token tiles of a unit are given launch
-    // indices b = 8 k + (unit mod 8) and share one XCD's L2: the weights come
-    // from memory once instead of once per XCD.  Units past the last multiple
-    // of 8 keep the plain order.
-    int tt, unit;
-    {
-        const int nt = gridDim.x;
-        const int b = blockIdx.x + nt * (blockIdx.y + gridDim.y * blockIdx.z);
-        const int units8 = (gridDim.y * gridDim.z) & ~7;
-        if (b < units8 * nt) {
-            const int k = b >> 3;
-            unit = (k / nt) * 8 + (b & 7);
-            tt = k % nt;
-        } else {
-            const int b2 = b - units8 * nt;
-            unit = units8 + b2 / nt;
-            tt = b2 % nt;
-        }
-    }
-    const int split = unit / static_cast<int>(gridDim.y);
-    const int t0 = tt * BT, r0 = (unit - split * static_cast<int>(gridDim.y)) * BR;
-    const int G = a.cols >> 6, gl = G - 1;
-    // this block's column groups: [g0, g1) of K split `split`
-    const int g0 = split * a.gps, g1 = min(G, g0 + a.gps), glast = g1 - 1;
-    const uint32_t row_bytes = static_cast<uint32_t>(a.cols) >> 1;
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    const int q = lane >> 4, lr = lane & 15;
-    const int wr = (wid / WGT) * T::kWR, wt = (wid % WGT) * T::kWT;
-    // A operand: byte offsets of this lane's 8 bytes in each tile row (rows past the end read the
-    // last row); the half-1 offset depends on the chunk's group count, full or the last chunk's
-    const __amdgpu_buffer_rsrc_t nib_r = buf_rsrc(a.nib, static_cast<uint32_t>(a.rows) * row_bytes);
-    const int lastc = gl >> 6;
-    const uint32_t gc_full = static_cast<uint32_t>(min(64, G)), gc_last = static_cast<uint32_t>(G - (lastc << 6));
-    uint32_t aoff_full[TI], aoff_last[TI];
-#pragma unroll
-    for (int i = 0; i < TI; ++i) {
-        const uint32_t base =
-            static_cast<uint32_t>(min(r0 + wr + 16 * i + lr, a.rows - 1)) * row_bytes + (q & 1) * 8u;
-        aoff_full[i] = base + static_cast<uint32_t>(q >> 1) * gc_full * 16u;
-        aoff_last[i] = base + static_cast<uint32_t>(q >> 1) * gc_last * 16u;
-    }
-    // x staging: piece j of this thread is token (tid >> 4) + kTokStep j, 16 bytes at (tid & 15) of
-    // the token's 256-byte LDS row (x_hi columns 0..63, then x_lo)
-    const __amdgpu_buffer_rsrc_t x_r = buf_rsrc(a.xh, static_cast<uint32_t>(a.m_pad) * a.cols * 4u);
-    const int xtok = threadIdx.x >> 4, c16 = threadIdx.x & 15;
-    uint32_t xoff[XU];
-#pragma unroll
-    for (int j = 0; j < XU; ++j)
-        xoff[j] = (static_cast<uint32_t>((c16 >> 3) * a.m_pad + t0 + xtok + j * kTokStep) * a.cols +
-                   (c16 & 7) * 8u) * 2u;
-    const int xdst = xtok * kGemmXLd + c16 * 8;
-    // scales: thread < BR stages row r0 + tid (the others load out of range: zero, no branch)
-    const __amdgpu_buffer_rsrc_t meta_r =
-        buf_rsrc(a.meta, meta_total_bytes<META>(static_cast<uint32_t>(a.rows), static_cast<uint32_t>(G)));
-    const bool s_thread = threadIdx.x < BR;
-    const uint32_t moff =
-        s_thread ? static_cast<uint32_t>(min(r0 + static_cast<int>(threadIdx.x), a.rows - 1)) * G * kMetaBytes : kBufOOB;
-
-#define GEMM_LOAD_A(W, gg)                                                                                   \
-    {                                                                                                        \
-        const int g_ = (gg), c_ = g_ >> 6;                                                                   \
-        const uint32_t so_ = static_cast<uint32_t>(c_) * 2048u + static_cast<uint32_t>(g_ & 63) * 16u;       \
-        const bool last_ = c_ == lastc;                                                                      \
-        _Pragma("unroll") for (int i_ = 0; i_ < TI; ++i_) W[i_] = __builtin_amdgcn_raw_buffer_load_b64(      \
-            nib_r, last_ ? aoff_last[i_] : aoff_full[i_], so_, 0);                                            \
-    }
-#define GEMM_LOAD_X(X, M, gg)                                                                                \
-    {                                                                                                        \
-        const uint32_t g_ = static_cast<uint32_t>(gg);                                                       \
-        _Pragma("unroll") for (int j_ = 0; j_ < XU; ++j_) X[j_] =                                            \
-            __builtin_amdgcn_raw_buffer_load_b128(x_r, xoff[j_], g_ * 128u, 0);                              \
-        M = META == 2 ? static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(meta_r, moff, g_ * kMetaBytes, 0)) \
-                      : __builtin_amdgcn_raw_buffer_load_b32(meta_r, moff, g_ * kMetaBytes, 0);                \
-    }
-#define GEMM_STORE_X(X, M, st)                                                                               \
-    {                                                                                                        \
-        _Float16* d_ = xlds + (st) * T::kXStage + xdst;                                                      \
-        _Pragma("unroll") for (int j_ = 0; j_ < XU; ++j_) *reinterpret_cast<u32x4*>(d_ + j_ * kTokStep * kGemmXLd) = \
-            X[j_];                                                                                           \
-        if (s_thread) slds[(st) * BR + threadIdx.x] = META == 1 || META == 3 ? __uint_as_float(M) : half_lo(M); \
-    }
-// MFMAs of one group, each tile's four chained into a per-group sum that is scaled into acc
-#define GEMM_COMPUTE(st, W)                                                                                  \
-    {                                                                                                        \
-        const _Float16* xs_ = xlds + (st) * T::kXStage;                                                      \
-        half8 bh_[TJ][2], bl_[TJ][2];                                                                        \
-        _Pragma("unroll") for (int j_ = 0; j_ < TJ; ++j_) {                                                  \
-            _Pragma("unroll") for (int k_ = 0; k_ < 2; ++k_) {                                               \
-                const int o_ = (wt + 16 * j_ + lr) * kGemmXLd + (2 * q + k_) * 8;                            \
-                bh_[j_][k_] = *reinterpret_cast<const half8*>(xs_ + o_);                                     \
-                bl_[j_][k_] = *reinterpret_cast<const half8*>(xs_ + o_ + 64);                                \
-            }                                                                                                \
-        }                                                                                                    \
-        _Pragma("unroll") for (int i_ = 0; i_ < TI; ++i_) {                                                  \
-            const floatx4 sv_ = *reinterpret_cast<const floatx4*>(slds + (st) * BR + wr + 16 * i_ + 4 * q);  \
-            const half8 a0_ = codes_to_h8(W[i_].x), a1_ = codes_to_h8(W[i_].y);                              \
-            _Pragma("unroll") for (int j_ = 0; j_ < TJ; ++j_) {                                              \
-                floatx4 t_ = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0_, bh_[j_][0], zero4, 0, 0, 0);        \
-                t_ = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0_, bl_[j_][0], t_, 0, 0, 0);                   \
-                t_ = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1_, bh_[j_][1], t_, 0, 0, 0);                   \
-                t_ = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1_, bl_[j_][1], t_, 0, 0, 0);                   \
-                _Pragma("unroll") for (int v_ = 0; v_ < 4; ++v_) acc[i_][j_][v_] =                           \
-                    fmaf(sv_[v_], t_[v_], acc[i_][j_][v_]);                                                  \
-            }                                                                                                \
-        }                                                                                                    \
-    }
-// step U of four: MFMAs of group g + U (LDS stage U & 1, A ring slot W), refill W with
-// group g + U + 4, store the x piece X (group g + U + 1) to the other stage, refill X
-// with group g + U + 3.  Loads past the last group re-read it, so every step issues the
-// same loads and the wait counts stay exact.
-#define GEMM_STEP(U, W, X, M)                                                                                \
-    {                                                                                                        \
-        const int gg_ = g + (U);                                                                             \
-        if (gg_ < g1) GEMM_COMPUTE((U) & 1, W);                                                              \
-        GEMM_LOAD_A(W, min(gg_ + 4, glast));                                                                 \
-        GEMM_STORE_X(X, M, ((U) + 1) & 1);                                                                   \
-        GEMM_LOAD_X(X, M, min(gg_ + 3, glast));                                                              \
-        __syncthreads();                                                                                     \
-    }
-
-    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    floatx4 acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = zero4;
-    u32x2 wa0[TI], wa1[TI], wa2[TI], wa3[TI];
-    u32x4 xa[XU], xb[XU];  // x pieces of the even / odd groups
-    uint32_t ma = 0, mb = 0;
-    GEMM_LOAD_A(wa0, g0);
-    GEMM_LOAD_A(wa1, min(g0 + 1, glast));
-    GEMM_LOAD_A(wa2, min(g0 + 2, glast));
-    GEMM_LOAD_A(wa3, min(g0 + 3, glast));
-    GEMM_LOAD_X(xa, ma, g0);
-    GEMM_LOAD_X(xb, mb, min(g0 + 1, glast));
-    GEMM_STORE_X(xa, ma, 0);
-    GEMM_LOAD_X(xa, ma, min(g0 + 2, glast));
-    __syncthreads();
-    for (int g = g0; g < g1; g += 4) {
-        GEMM_STEP(0, wa0, xb, mb);
-        GEMM_STEP(1, wa1, xa, ma);
-        GEMM_STEP(2, wa2, xb, mb);
-        GEMM_STEP(3, wa3, xa, ma);
-    }
-#undef GEMM_STEP
-#undef GEMM_COMPUTE
-#undef GEMM_STORE_X
-#undef GEMM_LOAD_X
-#undef GEMM_LOAD_A
-    // c0 term: K = G, lane group q takes groups gb + 8 q + 0..7 of its row / token.  All loads of a
-    // chunk are issued before any use; groups past G read out of range (zero), so c0 and xs are 0.
-    const __amdgpu_buffer_rsrc_t xs_r = buf_rsrc(a.xs, static_cast<uint32_t>(a.m_pad) * G * 4u);
-    for (int gb = g0; gb < (a.zero_is_8 ? g0 : g1); gb += 32) {
-        const int g8 = gb + 8 * q;
-        MetaWord<META> mw[TI][8];
-        uint32_t xw[TJ][8];
-#pragma unroll
-        for (int i = 0; i < TI; ++i) {
-            const uint32_t row = static_cast<uint32_t>(min(r0 + wr + 16 * i + lr, a.rows - 1));
-            const uint32_t off = (row * G + static_cast<uint32_t>(g8)) * kMetaBytes;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const bool in = g8 + e < g1;
-                const uint32_t o = in ? off + kMetaBytes * e : kBufOOB;
-                const uint32_t zo =
-                    META == 3 && in ? z4_offset(static_cast<uint32_t>(a.rows), static_cast<uint32_t>(G), row,
-                                                static_cast<uint32_t>(g8 + e))
-                                    : kBufOOB;
-                mw[i][e] = load_meta<META, 0>(meta_r, o, zo);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const uint32_t off = (static_cast<uint32_t>(t0 + wt + 16 * j + lr) * G + static_cast<uint32_t>(g8)) * 4u;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                xw[j][e] = __builtin_amdgcn_raw_buffer_load_b32(xs_r, g8 + e < g1 ? off + 4u * e : kBufOOB, 0, 0);
-        }
-        half8 ch[TI], cl[TI], sh[TJ], sl[TJ];
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float sc = meta_scale(mw[i][e]);
-                const float z = meta_zero_at(mw[i][e], static_cast<uint32_t>((g8 + e) & 7) * 4u);
-                const float c0 = 64.0f * (a.affine ? fmaf(8.0f, sc, z) : (8.0f - z) * sc);
-                ch[i][e] = static_cast<_Float16>(c0);
-                cl[i][e] = static_cast<_Float16>(c0 - static_cast<float>(ch[i][e]));
-            }
-#pragma unroll
-        for (int j = 0; j < TJ; ++j)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v = __builtin_bit_cast(float, xw[j][e]) * 0.015625f;
-                sh[j][e] = static_cast<_Float16>(v);
-                sl[j][e] = static_cast<_Float16>(v - static_cast<float>(sh[j][e]));
-            }
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cl[i], sh[j], acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ch[i], sl[j], acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ch[i], sh[j], acc[i][j], 0, 0, 0);
-            }
-    }
-
-    // epilogue: lane holds rows 4 (lane >> 4) + v of tile i, token (lane & 15) of tile j
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const int t = t0 + wt + j * 16 + lr;
-            const int rb = r0 + wr + i * 16 + 4 * q;
-            if (t >= a.m) continue;
-            const float tsc = a.ts[t];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[i][j][v] *= tsc;
-            if (a.part) {  // K split: this split's partial products, the reduce applies the epilogue
-                float* pr = a.part + (static_cast<size_t>(split) * a.m + t) * a.rows;
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (rb + v < a.rows) pr[rb + v] = acc[i][j][v];
-                continue;
-            }
-            float* yr = a.y + static_cast<size_t>(t) * a.ldy;
-            if constexpr (EPI == 2) {  // interleaved (gate, up) rows -> silu(gate) * up
-#pragma unroll
-                for (int v = 0; v < 4; v += 2)
-                    if (rb + v + 1 < a.rows) yr[(rb + v) >> 1] = silu_dev(acc[i][j][v]) * acc[i][j][v + 1];
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    if (rb + v >= a.rows) continue;
-                    if constexpr (EPI == 1)
-                        yr[rb + v] += acc[i][j][v];
-                    else
-                        yr[rb + v] = acc[i][j][v];
-                }
-            }
-        }
-}
-
-// The launch's tile (gemm_w4_mfma_kernel<4, 1, 2, 4, ...>): 128 rows x 64 tokens.
-constexpr int kGemmBR = 128, kGemmBT = 64;
-constexpr int kGemmMaxSplits = 4;
-
-// K splits of a launch: with fewer than two blocks per CU (the 4096-row
-// projections of a 512-token chunk: 256 blocks) the column groups are split
-// over blockIdx.z, each split keeping at least 16 groups, and a second kernel
-// adds the splits' partial products in a fixed order (deterministic).  The
-// SiLU-pair epilogue (gate/up, 1536 blocks) is never split.
-static int gemm_splits(int rows, int m, int cols, int epi) {
-    if (epi == 2) return 1;
-    const int blocks = ((m + kGemmBT - 1) / kGemmBT) * ((rows + kGemmBR - 1) / kGemmBR);
-    const int G = cols / 64;
-    int splits = 1;
-    while (splits < kGemmMaxSplits && blocks * splits < 2 * 256 && G / (2 * splits) >= 16) splits *= 2;
-    return splits;
-}
-
-static size_t gemm_prep_bytes(int m, int cols) {
-    const size_t m_pad = static_cast<size_t>((m + kGemmPad - 1) / kGemmPad) * kGemmPad;
-    return m_pad * static_cast<size_t>(cols) * (2 * sizeof(_Float16)) +
-           m_pad * static_cast<size_t>(cols / 64) * sizeof(float) + m_pad * sizeof(float);
-}
-
-// A bound that grows with m and with rows, so that a workspace sized for a
-// chunk's most tokens and widest matrix serves every smaller call: the partial
-// products of a split launch (fewer tokens or rows can split into more) never
-// exceed kGemmMaxSplits m rows, nor the tiles of fewer than 2 x 512 blocks.
-size_t gemm_workspace_bytes(int m, int cols, int rows) {
-    const size_t all = static_cast<size_t>(kGemmMaxSplits) * m * std::max(0, rows);
-    const size_t part = std::min<size_t>(all, size_t{2 * 512} * kGemmBR * kGemmBT) * sizeof(float);
-    return gemm_prep_bytes(m, cols) + (part + 255) / 256 * 256;
-}
-
-// y[t][r] (op)= sum over splits z (in order) of part[z][t][r]; op: store, add
-__global__ void __launch_bounds__(256) gemm_splitk_reduce_kernel(const float* __restrict__ part, int splits, int m,
-                                                                 int rows, float* __restrict__ y, int ldy, int add) {
-    const size_t n = static_cast<size_t>(m) * rows;
-    const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-        float v = part[i];
-        for (int z = 1; z < splits; ++z) v += part[static_cast<size_t>(z) * n + i];
-        const size_t t = i / rows, r = i - t * rows;
-        float* yp = y + t * ldy + r;
-        *yp = add ? *yp + v : v;
-    }
-}
-
-bool gemm_supported(int rows, int cols, int group, int layout, const Prologue& pro) {
-    if ((layout != 0 && layout != 2 && layout != 3 && layout != 4) || group != 64 || cols % 64 != 0 || cols / 64 > 256 ||
-        rows <= 0)
-        return false;
-    if (pro.mode == PRO_GATED)
-        return pro.head_dim > 0 && pro.head_dim % 8 == 0 && cols % pro.head_dim == 0 &&
-               cols / pro.head_dim <= kPrepMaxHeads;
-    return true;
-}
-
-template <int WGR, int WGT, int TI, int TJ, int EPI, int META>
-static hipError_t launch_gemm_cfg(const GemmArgs& a, int splits, hipStream_t s) {
-    using T = GemmTile<WGR, WGT, TI, TJ>;
-    const auto fn = reinterpret_cast<const void*>(&gemm_w4_mfma_kernel<WGR, WGT, TI, TJ, EPI, META>);
-    if constexpr (T::kLds > 64 * 1024) {  // beyond the default dynamic-LDS limit (gfx950 has 160 KiB per CU)
-        if (hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(T::kLds));
-            e != hipSuccess)
-            return e;
-    }
-    static_assert(T::kBR == kGemmBR && T::kBT == kGemmBT, "split choice assumes this tile");
-    const dim3 grid((a.m + T::kBT - 1) / T::kBT, (a.rows + T::kBR - 1) / T::kBR, splits);
-    hipLaunchKernelGGL((gemm_w4_mfma_kernel<WGR, WGT, TI, TJ, EPI, META>), grid, dim3(T::kThreads), T::kLds, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_gemm(const GemmLaunch& p, hipStream_t s) {
-    const int m_pad = (p.m + kGemmPad - 1) / kGemmPad * kGemmPad;
-    _Float16* xh = static_cast<_Float16*>(p.workspace);
-    _Float16* xl = xh + static_cast<size_t>(m_pad) * p.cols;
-    float* xs = reinterpret_cast<float*>(xl + static_cast<size_t>(m_pad) * p.cols);
-    float* ts = xs + static_cast<size_t>(m_pad) * (p.cols / 64);
-    const int nk = p.cols / 2048;
-    const bool vec = prep_vec_ok(p) && (nk == 1 || nk == 2 || nk == 6) &&
-                     (nk == 1 ? launch_prep_vec<1>(p, m_pad, xh, xl, xs, ts, s)
-                              : nk == 2 ? launch_prep_vec<2>(p, m_pad, xh, xl, xs, ts, s)
-                                        : launch_prep_vec<6>(p, m_pad, xh, xl, xs, ts, s));
-    if (!vec)
-        hipLaunchKernelGGL(prep_x_kernel, dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.cols, p.pro, p.ldz, xh, xl,
-                           xs, ts);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    const int splits = gemm_splits(p.rows, p.m, p.cols, p.epi);
-    const int G = p.cols / 64;
-    float* part = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(p.workspace) +
-                                                        gemm_prep_bytes(m_pad, p.cols)) : nullptr;
-    GemmArgs a{p.nib, static_cast<const uint32_t*>(p.meta), p.rows, p.cols, p.affine, p.zero_is_8, xh, xs, ts,
-               (G + splits - 1) / splits, part, p.m, m_pad, p.y, p.ldy};
-    // 128 rows x 64 tokens per block: four waves of 32 rows x 64 tokens
-    // metadata form: 0 fp16 (scale, zero), 1 fp32 pair (layout 2), 2 fp16 scale, zero 8 (layout 3),
-    // 3 fp32 scale and 4-bit zero (layout 4)
-    const int meta = p.layout == 2 ? 1 : (p.layout == 3 ? 2 : (p.layout == 4 ? 3 : 0));
-    hipError_t e = hipErrorInvalidValue;
-    switch (p.epi * 4 + meta) {
-        case 0: e = launch_gemm_cfg<4, 1, 2, 4, 0, 0>(a, splits, s); break;
-        case 1: e = launch_gemm_cfg<4, 1, 2, 4, 0, 1>(a, splits, s); break;
-        case 2: e = launch_gemm_cfg<4, 1, 2, 4, 0, 2>(a, splits, s); break;
-        case 3: e = launch_gemm_cfg<4, 1, 2, 4, 0, 3>(a, splits, s); break;
-        case 4: e = launch_gemm_cfg<4, 1, 2, 4, 1, 0>(a, splits, s); break;
-        case 5: e = launch_gemm_cfg<4, 1, 2, 4, 1, 1>(a, splits, s); break;
-        case 6: e = launch_gemm_cfg<4, 1, 2, 4, 1, 2>(a, splits, s); break;
-        case 7: e = launch_gemm_cfg<4, 1, 2, 4, 1, 3>(a, splits, s); break;
-        case 8: e = launch_gemm_cfg<4, 1, 2, 4, 2, 0>(a, splits, s); break;
-        case 9: e = launch_gemm_cfg<4, 1, 2, 4, 2, 1>(a, splits, s); break;
-        case 10: e = launch_gemm_cfg<4, 1, 2, 4, 2, 2>(a, splits, s); break;
-        case 11: e = launch_gemm_cfg<4, 1, 2, 4, 2, 3>(a, splits, s); break;
-        default: return hipErrorInvalidValue;
-    }
-    if (e != hipSuccess || splits == 1) return e;
-    const size_t n = static_cast<size_t>(p.m) * p.rows;
-    const int blocks = static_cast<int>(std::min<size_t>((n + 255) / 256, 2048));
-    hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3(blocks), dim3(256), 0, s, part, splits, p.m, p.rows, p.y,
-                       p.ldy, p.epi == 1 ? 1 : 0);
-    return hipGetLastError();
-}
 
 // ---------------------------------------------------------------------------
 // Linear attention over a prompt chunk: block (vh, 16-column slice) runs the
