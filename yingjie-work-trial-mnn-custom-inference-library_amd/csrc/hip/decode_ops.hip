@@ -12,6 +12,8 @@
 //   conv1d + SiLU           custom_model.cpp:961-1010
 //   L2-normalised heads     custom_model.cpp:315-327
 //   gated delta rule        custom_model.cpp:1074-1096, kernels/reference/ref_delta.cpp:8-41
+#include <algorithm>
+
 #include "xqhip_common.hpp"
 #include "xqhip_kernels.hpp"
 #include "linear_step.hpp"
@@ -703,8 +705,11 @@ static size_t gqa_lds_bytes(int group, int head_dim) {
 
 static int combine_threads(int head_dim) { return min(256, max(64, ((head_dim + 63) / 64) * 64)); }
 
+static hipError_t launch_attn_decode_wide(const AttnDecodeLaunch& a, hipStream_t s);
+
 hipError_t launch_attn_decode(const AttnDecodeLaunch& a, hipStream_t s) {
     const GqaLaunch& p = a.g;
+    if (p.head_dim == 256) return launch_attn_decode_wide(a, s);
     const int group = p.nq / p.nkv;
     const size_t lds = gqa_lds_bytes(group, p.head_dim) + 2 * sizeof(float) * p.head_dim;
     const int slots = attn_slots(p.nkv);
@@ -712,7 +717,6 @@ hipError_t launch_attn_decode(const AttnDecodeLaunch& a, hipStream_t s) {
     switch (attn_hd_class(p.head_dim)) {
         case 64: hipLaunchKernelGGL(attn_decode_kernel<64>, grid, dim3(kAttnThreads), lds, s, a); break;
         case 128: hipLaunchKernelGGL(attn_decode_kernel<128>, grid, dim3(kAttnThreads), lds, s, a); break;
-        case 256: hipLaunchKernelGGL(attn_decode_kernel<256>, grid, dim3(kAttnThreads), lds, s, a); break;
         default: hipLaunchKernelGGL(attn_decode_kernel<0>, grid, dim3(kAttnThreads), lds, s, a); break;
     }
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
@@ -760,8 +764,10 @@ constexpr int kHeadThreads = 512;
 constexpr int kHeadPass = 1024;                    // tokens per pass
 constexpr int kHeadKSub = kHeadThreads / 4;        // tokens per K sub-pass (128)
 constexpr int kHeadKSubs = kHeadPass / kHeadKSub;  // 8
-constexpr int kHeadVTok = kHeadThreads / 16;       // tokens per V sub-pass (32)
-constexpr int kHeadVPerK = kHeadKSub / kHeadVTok;  // V sub-passes per K sub-pass (4)
+// value lanes per token (8 dims each), tokens per V sub-pass, V sub-passes per K sub-pass
+template <int HD> constexpr int kHeadVLanes = HD / 8;
+template <int HD> constexpr int kHeadVTok = kHeadThreads / kHeadVLanes<HD>;
+template <int HD> constexpr int kHeadVPerK = kHeadKSub / kHeadVTok<HD>;
 
 template <int HD>
 struct HeadSmem {
@@ -796,21 +802,24 @@ __device__ __forceinline__ void wave_lds_sync() {
 // A pass is kHeadPass tokens for the per-head kernel and half that for the
 // split kernel (whose ranges are an eighth of the context), which keeps the
 // split kernel's longest body within the register file.
-// kPassSubs(PART): 128-token sub-passes per pass
-template <bool PART>
-constexpr int kPassSubs = PART ? kHeadKSubs / 2 : kHeadKSubs;
+// kPassSubs: 128-token sub-passes per pass
+template <int HD, bool PART>
+constexpr int kPassSubs = PART ? kHeadKSubs * 64 / HD : kHeadKSubs;
 
 template <int HD, int KS, bool PART>
 __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSmem<HD>& sm, int pos, int c0, int c1,
                                                bool fresh, float* part_out) {
-    static_assert(HD == 128, "4 score lanes x 32 dims, 16 value lanes x 8 dims");
+    static_assert(HD == 128 || (HD == 256 && PART), "4 score lanes x HD / 4 dims, HD / 8 value lanes x 8 dims");
     constexpr int kWaves = kHeadThreads / kWave;
-    constexpr int kSubs = kPassSubs<PART>;
+    constexpr int kSubs = kPassSubs<HD, PART>;
+    constexpr int KU = HD / 32;            // 16-byte pieces of a key per score lane
+    constexpr int NV = HD / kWave;         // dims per lane of the waves that prepare q, k and v
+    constexpr int VL = kHeadVLanes<HD>, VT = kHeadVTok<HD>, VPK = kHeadVPerK<HD>;
     constexpr int kPass = kSubs * kHeadKSub;  // tokens per pass
     static_assert(KS >= 1 && KS <= kSubs, "first-pass sub-passes");
     // the first pass's values are requested with its keys when both fit the
-    // register budget beside each other (up to 512 tokens)
-    constexpr bool kVPre = KS <= 4;
+    // register budget beside each other (up to 512 tokens of 128 dims)
+    constexpr bool kVPre = KS * HD <= 512;
     const GqaLaunch& p = a.g;
     const int group = p.nq / p.nkv;
     // blocks b, b + nkv, b + 2 nkv, ... take the query heads of one kv head:
@@ -821,7 +830,7 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
     const bool owner = fresh && qh % group == 0;  // appends the new key / value of kv head kh
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
     const int sub = tid & 3, tt = tid >> 2;   // score lanes: dims 32 u + 8 sub + e of token tt
-    const int dsl = tid & 15, ts = tid >> 4;  // value lanes: dims 8 dsl + e of token ts
+    const int dsl = tid % VL, ts = tid / VL;  // value lanes: dims 8 dsl + e of token ts
     const float rscale = 1.0f / sqrtf(static_cast<float>(HD));
     const size_t kv_stride = static_cast<size_t>(p.nkv) * HD;
     const uint32_t row_bytes = static_cast<uint32_t>(kv_stride) * 2u;  // one position of a cache
@@ -830,14 +839,22 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
     const float* src = wid == 0 ? a.q_src + static_cast<size_t>(qh) * (a.gated ? 2 * HD : HD)
                                 : (wid == 1 ? a.k_src : a.v_src) + static_cast<size_t>(kh) * HD;
     const float* nw = wid == 0 ? a.q_norm : a.k_norm;
-    const float hv0 = src[lane], hv1 = src[lane + kWave];
-    const float w0 = nw[lane], w1 = nw[lane + kWave];
-    const int half = a.rotary_dim / 2;  // <= HD / 2 = kWave: one rotary pair per lane of waves 0 and 1
+    float hv[NV], nwv[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        hv[i] = src[lane + kWave * i];
+        nwv[i] = nw[lane + kWave * i];
+    }
+    const int half = a.rotary_dim / 2;  // <= HD / 2: NV / 2 rotary pairs per lane of waves 0 and 1
     const __amdgpu_buffer_rsrc_t r_cs =
         buf_rsrc(a.rope_cs, half > 0 ? static_cast<uint32_t>(pos + 1) * a.rope_pairs * 8u : 0u);
-    const uint32_t cs_off =
-        wid < 2 && lane < half ? (static_cast<uint32_t>(pos) * a.rope_pairs + lane) * 8u : kBufOOB;
-    const auto csw = __builtin_amdgcn_raw_buffer_load_b64(r_cs, cs_off, 0, 0);
+    u32x2 csw[NV / 2];
+#pragma unroll
+    for (int i = 0; i < NV / 2; ++i) {
+        const int d = lane + kWave * i;
+        const uint32_t cs_off = wid < 2 && d < half ? (static_cast<uint32_t>(pos) * a.rope_pairs + d) * 8u : kBufOOB;
+        csw[i] = __builtin_amdgcn_raw_buffer_load_b64(r_cs, cs_off, 0, 0);
+    }
     // no gate projection: the reference's zero gate, sigmoid(0) (custom_model.cpp:750-753)
     const __amdgpu_buffer_rsrc_t r_gate =
         buf_rsrc(p.gate, p.gate ? static_cast<uint32_t>(p.nq) * p.gate_stride * 4u : 0u);
@@ -851,21 +868,21 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
 #pragma unroll
         for (int j = 0; j < J; ++j)
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < KU; ++u)
                 kr[j][u] = buf_load_u4(r, static_cast<uint32_t>(tt + kHeadKSub * j) * row_bytes + sub * 16u + u * 64u);
     };
     // the values of cached positions [t0, t0 + nc), rows past nc read 0: value
-    // sub-pass jj (32 tokens) of this thread is token ts + 32 jj
+    // sub-pass jj (VT tokens) of this thread is token ts + VT jj
     auto load_v = [&](int t0, int nc, auto& vr) {
         constexpr int JV = sizeof(vr) / sizeof(vr[0]);
         const __amdgpu_buffer_rsrc_t r = buf_rsrc(p.v_cache + static_cast<size_t>(t0) * kv_stride + kh * HD,
                                                   static_cast<uint32_t>(nc) * row_bytes);
 #pragma unroll
         for (int jj = 0; jj < JV; ++jj)
-            vr[jj] = buf_load_u4(r, static_cast<uint32_t>(ts + kHeadVTok * jj) * row_bytes + dsl * 16u);
+            vr[jj] = buf_load_u4(r, static_cast<uint32_t>(ts + VT * jj) * row_bytes + dsl * 16u);
     };
-    uint4 kr[KS][4];
-    uint4 vpre[kVPre ? KS * kHeadVPerK : 1];
+    uint4 kr[KS][KU];
+    uint4 vpre[kVPre ? KS * VPK : 1];
     load_k(c0, min(kPass, c1 - c0), kr);
     if constexpr (kVPre) load_v(c0, min(kPass, c1 - c0), vpre);
     // per-head RMSNorm (custom_model.cpp:301-313) of q (wave 0) and k (wave 1),
@@ -875,50 +892,57 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
     // rounded, like every slot, appended by the kv head's first query head
     const size_t slot = static_cast<size_t>(pos) * kv_stride + static_cast<size_t>(kh) * HD;
     if (wid < 2) {
-        float ss = hv0 * hv0 + hv1 * hv1;
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) ss += hv[i] * hv[i];
         ss = wave_sum(ss);
         const float inv = 1.0f / sqrtf(ss / static_cast<float>(HD) + a.eps);
         float* dst = wid == 0 ? sm.qs : sm.kn;
-        dst[lane] = hv0 * (inv * w0);
-        dst[lane + kWave] = hv1 * (inv * w1);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) dst[lane + kWave * i] = hv[i] * (inv * nwv[i]);
         wave_lds_sync();
-        if (lane < half) {
-            const float cx = __uint_as_float(csw[0]), cy = __uint_as_float(csw[1]);
-            const float x0 = dst[lane], x1 = dst[half + lane];
-            dst[lane] = x0 * cx - x1 * cy;
-            dst[half + lane] = x1 * cx + x0 * cy;
+#pragma unroll
+        for (int i = 0; i < NV / 2; ++i) {  // the pairs (d, half + d) are disjoint
+            const int d = lane + kWave * i;
+            if (d < half) {
+                const float cx = __uint_as_float(csw[i][0]), cy = __uint_as_float(csw[i][1]);
+                const float x0 = dst[d], x1 = dst[half + d];
+                dst[d] = x0 * cx - x1 * cy;
+                dst[half + d] = x1 * cx + x0 * cy;
+            }
         }
         if (wid == 1) {
             wave_lds_sync();
-            const _Float16 k0 = static_cast<_Float16>(sm.kn[lane]), k1 = static_cast<_Float16>(sm.kn[lane + kWave]);
-            if (owner) {
-                a.k_cache[slot + lane] = k0;
-                a.k_cache[slot + lane + kWave] = k1;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const _Float16 k0 = static_cast<_Float16>(sm.kn[lane + kWave * i]);
+                if (owner) a.k_cache[slot + lane + kWave * i] = k0;
+                sm.kn[lane + kWave * i] = static_cast<float>(k0);
             }
-            sm.kn[lane] = static_cast<float>(k0);
-            sm.kn[lane + kWave] = static_cast<float>(k1);
         }
     } else if (wid == 2) {
-        const _Float16 v0 = static_cast<_Float16>(hv0), v1 = static_cast<_Float16>(hv1);
-        if (owner) {
-            a.v_cache[slot + lane] = v0;
-            a.v_cache[slot + lane + kWave] = v1;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const _Float16 v0 = static_cast<_Float16>(hv[i]);
+            if (owner) a.v_cache[slot + lane + kWave * i] = v0;
+            sm.vn[lane + kWave * i] = static_cast<float>(v0);
         }
-        sm.vn[lane] = static_cast<float>(v0);
-        sm.vn[lane + kWave] = static_cast<float>(v1);
     }
     if (tid < HD) sm.gate[tid] = gv;
     __syncthreads();
     // q in registers, in the score lanes' dim order
-    float qreg[32];
+    float qreg[8 * KU];
 #pragma unroll
-    for (int d = 0; d < 32; ++d) qreg[d] = sm.qs[(d >> 3) * 32 + sub * 8 + (d & 7)];
+    for (int d = 0; d < 8 * KU; ++d) qreg[d] = sm.qs[(d >> 3) * 32 + sub * 8 + (d & 7)];
     // the new token's score (the last wave; pos lies in the last pass)
     if (wid == kWaves - 1) {
-        float s = sm.qs[lane] * sm.kn[lane] + sm.qs[lane + kWave] * sm.kn[lane + kWave];
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) s += sm.qs[lane + kWave * i] * sm.kn[lane + kWave * i];
         s = wave_sum(s);
         if (lane == 0) sm.fresh_s = s * rscale;
     }
+    constexpr bool kExpOnce = HD == 256;  // see the value sum
     float run_m = -INFINITY, l = 0.0f, o[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = 0.0f;
@@ -939,7 +963,7 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
             const int tl = tt + kHeadKSub * j;
             float dot = 0.0f;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < KU; ++u) {
                 const uint32_t ww[4] = {kp[j][u].x, kp[j][u].y, kp[j][u].z, kp[j][u].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -955,9 +979,9 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
             // the values of these 128 tokens, into the registers the keys held
             if constexpr (!kLoaded) {
 #pragma unroll
-                for (int r = 0; r < kHeadVPerK; ++r) {
-                    const int jj = kHeadVPerK * j + r;
-                    vr[jj] = buf_load_u4(r_v, static_cast<uint32_t>(ts + kHeadVTok * jj) * row_bytes + dsl * 16u);
+                for (int r = 0; r < VPK; ++r) {
+                    const int jj = VPK * j + r;
+                    vr[jj] = buf_load_u4(r_v, static_cast<uint32_t>(ts + VT * jj) * row_bytes + dsl * 16u);
                 }
             }
         }
@@ -973,13 +997,27 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] *= f_old;
         run_m = mn;
-        // sum_t exp(s_t - m) v_t over this thread's tokens ts, ts + 32, ...
+        // exp(s_t - m), once per token (positions past the pass's last weigh 0), where a token's HD / 8 value lanes
+        // repeating it cost more than the barrier (256 dims)
+        if constexpr (kExpOnce) {
 #pragma unroll
-        for (int jj = 0; jj < J * kHeadVPerK; ++jj) {
-            const int tl = ts + kHeadVTok * jj;
-            if (tl < nc) {
-                const float pr = expf(sm.sc[tl] - mn);
-                l += pr;
+            for (int k = 0; k < (J * kHeadKSub + kHeadThreads - 1) / kHeadThreads; ++k) {
+                const int t = tid + kHeadThreads * k;
+                if (t < J * kHeadKSub) {
+                    const float pr = t < nc ? expf(sm.sc[t] - mn) : 0.0f;
+                    sm.sc[t] = pr;
+                    l += pr;
+                }
+            }
+            __syncthreads();
+        }
+        // sum_t exp(s_t - m) v_t over this thread's tokens ts, ts + VT, ...
+#pragma unroll
+        for (int jj = 0; jj < J * VPK; ++jj) {
+            const int tl = ts + VT * jj;
+            if (kExpOnce || tl < nc) {
+                const float pr = kExpOnce ? sm.sc[tl] : expf(sm.sc[tl] - mn);
+                if (!kExpOnce) l += pr;
                 o[0] += pr * half_lo(vr[jj].x);
                 o[1] += pr * half_hi(vr[jj].x);
                 o[2] += pr * half_lo(vr[jj].y);
@@ -992,33 +1030,40 @@ __device__ __forceinline__ void head_attention(const AttnDecodeLaunch& a, HeadSm
         }
         if (last && ts == 0) {  // the new token, once per dim slice
             const float pr = expf(sm.fresh_s - mn);
-            l += pr;
+            if (!kExpOnce || dsl == 0) l += pr;
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] += pr * sm.vn[dsl * 8 + e];
         }
         __syncthreads();  // sc and red are rewritten by the next pass
     };
+    // Ranges of more than one pass are read in full passes; the new token may
+    // open a pass of its own.
+    auto more = [&](int t0) { return fresh ? t0 <= c1 : t0 < c1; };
     if constexpr (kVPre) {
         pass(c0, kr, vpre, std::true_type{});
     } else {
-        uint4 vr[KS * kHeadVPerK];
+        uint4 vr[KS * VPK];
         pass(c0, kr, vr, std::false_type{});
     }
-    // longer ranges: further passes of kSubs sub-passes, each loading its
-    // keys first (kept apart from the first pass so that no key register lives
-    // across a value phase); the new token may open a pass of its own
-    for (int t0 = c0 + kPass; fresh ? t0 <= c1 : t0 < c1; t0 += kPass) {
-        uint4 kr2[kSubs][4];
-        uint4 vr2[kSubs * kHeadVPerK];
-        load_k(t0, min(kPass, c1 - t0), kr2);
-        pass(t0, kr2, vr2, std::false_type{});
-    }
-    // lanes with the same dsl: 4 per wave (16 apart), then the waves through LDS;
-    // l is the same in every dsl lane of a token group and reduces alongside
+    // further passes load their keys first (kept apart from the first pass so
+    // that no key register lives across a value phase); requesting a pass's keys
+    // and values during the pass before measured slower (8100 positions: 17.1
+    // against 15.5 us at 128 dims, 19.8 against 17.9 at 256)
+    if constexpr (KS == kSubs)
+        for (int t0 = c0 + kPass; more(t0); t0 += kPass) {
+            uint4 kr2[kSubs][KU];
+            uint4 vr2[kSubs * VPK];
+            load_k(t0, min(kPass, c1 - t0), kr2);
+            pass(t0, kr2, vr2, std::false_type{});
+        }
+    // lanes with the same dsl, VL apart, then the waves through LDS
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = xor_pair_sum<32>(xor_pair_sum<16>(o[e]));
-    l = xor_pair_sum<32>(xor_pair_sum<16>(l));
-    if (lane < 16) {
+    for (int e = 0; e < 8; ++e) {
+        if constexpr (VL == 16) o[e] = xor_pair_sum<16>(o[e]);
+        o[e] = xor_pair_sum<32>(o[e]);
+    }
+    l = kExpOnce ? wave_sum(l) : xor_pair_sum<32>(xor_pair_sum<16>(l));  // once: a part per thread, else per token lane
+    if (lane < VL) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sm.ored[wid][dsl * 8 + e] = o[e];
         if (lane == 0) sm.ored[wid][HD] = l;
@@ -1093,7 +1138,7 @@ __global__ void __launch_bounds__(kHeadThreads) attn_decode_part_kernel(AttnDeco
             __hip_atomic_store(out + 1, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     } else {
-        constexpr int kSubs = kPassSubs<true>;
+        constexpr int kSubs = kPassSubs<HD, true>;
         const int ks = max(1, (min(c1 - c0, kSubs * kHeadKSub) + kHeadKSub - 1) / kHeadKSub);
         switch (ks) {
             case 1: head_attention<HD, 1, true>(a, sm, pos, c0, c1, fresh, out); break;
@@ -1147,6 +1192,76 @@ __global__ void __launch_bounds__(kHeadThreads) attn_decode_part_kernel(AttnDeco
         a.g.out[static_cast<size_t>(qh) * HD + tid] = (acc * (1.0f / L)) * sigmoid_dev(g);
     }
     if (threadIdx.x == 0) __hip_atomic_store(cnt + qh * 32, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// 256-dim heads (attn_decode's two launches): block (query head, split) is
+// attn_decode_part_kernel's without the counter, its record [kWideStride] of the
+// workspace merged by attn_merge_kernel after the kernel boundary.  One block
+// per CU: 16 query heads in 16 splits.  What bounds it: a block's serial chain (q and
+// k prepared, scores, maximum, exp, value sum) and the merge's launch.  16 / 4 heads, 2000 positions: 6.9 + 3.7 us for the merge, against
+// 19.6 us in all for a block per (kv head, 31 positions) that took its four query heads in turn.
+constexpr int kWideHd = 256, kWideMaxSplits = 32;
+constexpr int kWideStride = 288;  // floats per record: m, l, 2 pad, o[256], pad to whole 128-byte lines
+static_assert(kWideMaxSplits * kWideStride <= kAttnMaxSlots * (kWideHd + 2), "the slot workspace holds the records");
+
+__global__ void __launch_bounds__(kHeadThreads) attn_decode_wide_kernel(AttnDecodeLaunch a, float* part) {
+    __shared__ HeadSmem<kWideHd> sm;
+    const int pos = *a.g.pos;
+    const int splits = static_cast<int>(gridDim.y), sp = static_cast<int>(blockIdx.y);
+    const int per = (pos + splits - 1) / splits;
+    const int c0 = min(pos, sp * per), c1 = min(pos, c0 + per);
+    const bool fresh = sp == splits - 1;
+    const int qh = static_cast<int>(blockIdx.x) % a.g.nkv * (a.g.nq / a.g.nkv) + static_cast<int>(blockIdx.x) / a.g.nkv;
+    float* out = part + (static_cast<size_t>(sp) * a.g.nq + qh) * kWideStride;
+    if (!fresh && c0 == c1) {  // nothing cached in this range (block-uniform): an empty partial
+        if (threadIdx.x < kWideHd) out[kAttnPartO + threadIdx.x] = 0.0f;
+        if (threadIdx.x == 0) {
+            out[0] = -INFINITY;
+            out[1] = 0.0f;
+        }
+        return;
+    }
+    if (c1 - c0 <= kHeadKSub) head_attention<kWideHd, 1, true>(a, sm, pos, c0, c1, fresh, out);
+    else head_attention<kWideHd, kPassSubs<kWideHd, true>, true>(a, sm, pos, c0, c1, fresh, out);
+}
+
+template <int MAXS>
+__global__ void __launch_bounds__(kWideHd) attn_merge_kernel(GqaLaunch p, const float* part, int splits) {
+    const int qh = blockIdx.x, d = threadIdx.x;
+    // no gate projection: the reference's zero gate, sigmoid(0) (custom_model.cpp:750-753)
+    const float g = p.gate ? p.gate[static_cast<size_t>(qh) * p.gate_stride + d] : 0.0f;
+    float mv[MAXS], lv[MAXS], ov[MAXS], M = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < MAXS; ++s) {  // past the last split: its record again, weight 0 (every load in flight)
+        const float* q = part + (static_cast<size_t>(min(s, splits - 1)) * p.nq + qh) * kWideStride;
+        mv[s] = q[0];
+        lv[s] = q[1];
+        ov[s] = q[kAttnPartO + d];
+    }
+#pragma unroll
+    for (int s = 0; s < MAXS; ++s) {
+        if (s >= splits) mv[s] = -INFINITY;
+        M = fmaxf(M, mv[s]);
+    }
+    float L = 0.0f, acc = 0.0f;
+#pragma unroll
+    for (int s = 0; s < MAXS; ++s) {
+        const float w = expf(mv[s] - M);  // an empty range (m = -inf): 0
+        L += w * lv[s];
+        acc += w * ov[s];
+    }
+    p.out[static_cast<size_t>(qh) * kWideHd + d] = (acc * (1.0f / L)) * sigmoid_dev(g);
+}
+
+static hipError_t launch_attn_decode_wide(const AttnDecodeLaunch& a, hipStream_t s) {
+    const int splits = std::max(1, std::min(kWideMaxSplits, 256 / a.g.nq));
+    hipLaunchKernelGGL(attn_decode_wide_kernel, dim3(a.g.nq, splits), dim3(kHeadThreads), 0, s, a, a.g.part_m);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    if (splits <= 16)
+        hipLaunchKernelGGL(attn_merge_kernel<16>, dim3(a.g.nq), dim3(kWideHd), 0, s, a.g, a.g.part_m, splits);
+    else
+        hipLaunchKernelGGL(attn_merge_kernel<kWideMaxSplits>, dim3(a.g.nq), dim3(kWideHd), 0, s, a.g, a.g.part_m, splits);
+    return hipGetLastError();
 }
 
 bool attn_head_supported(int nq, int nkv, int head_dim) {
