@@ -280,9 +280,8 @@ __global__ void __launch_bounds__(256) prep_x_vec_kernel(const float* __restrict
     }
 }
 
-// the vectorised form's launch, or false when the shape or alignment needs the generic kernel
 template <int NK>
-static bool launch_prep_vec(const GemmLaunch& p, int m_pad, uint4* xt, float* xs, float* ts, hipStream_t s) {
+static void launch_prep_vec(const GemmLaunch& p, int m_pad, uint4* xt, float* xs, float* ts, hipStream_t s) {
     if (p.pro.mode == PRO_RMS)
         hipLaunchKernelGGL((prep_x_vec_kernel<NK, PRO_RMS>), dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.pro,
                            p.ldz, xt, xs, ts);
@@ -292,7 +291,6 @@ static bool launch_prep_vec(const GemmLaunch& p, int m_pad, uint4* xt, float* xs
     else
         hipLaunchKernelGGL((prep_x_vec_kernel<NK, PRO_NONE>), dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.pro,
                            p.ldz, xt, xs, ts);
-    return true;
 }
 
 static bool prep_vec_ok(const GemmLaunch& p) {
@@ -839,11 +837,26 @@ static GemmPlan gemm_plan(int rows, int m, int cols) {
     const int G = cols / 64;
     auto blocks = [&](int br, int bt) { return static_cast<long>((m + bt - 1) / bt) * ((rows + br - 1) / br); };
     GemmPlan p{};
+    p.splits = 1;
     long nb = blocks(128, 32);
     if (nb <= 600) {
         p.tile = kTileSmall;
         p.bt = 32;
-        p.splits = nb >= 136 ? 1 : static_cast<int>((520 / nb + 1) / 2);  // about 260 blocks
+        // Split while a group's time (us, for the blocks sharing a CU, as measured) times the groups left to a
+        // block outweighs the second kernel and the partial products' traffic.  2048x8192, 300 tokens (160 blocks):
+        // 46 us unsplit, 33 with 3.
+        auto per_group = [](double per_cu) {
+            return per_cu <= 1.0 ? 0.32 : per_cu <= 2.0 ? 0.12 + 0.2 * per_cu : per_cu <= 3.0 ? 0.28 * per_cu - 0.04 : 0.27 * per_cu;
+        };
+        double best = 1.0e30;
+        for (int s = 1; s <= std::min(kGemmMaxSplits, std::max(1, G / 8)); ++s) {
+            const double t = ((G + s - 1) / s + 3) / 4 * 4 * per_group(nb * s / 256.0) +
+                             (s > 1 ? 4.5 + 2.0e-6 * s * m * rows : 0.0);
+            if (t < best) {
+                best = t;
+                p.splits = s;
+            }
+        }
     } else {
         nb = blocks(256, 64);
         p.tile = nb > 256 && nb <= 512 ? kTileLarge : kTileMid;
@@ -866,11 +879,13 @@ hipError_t launch_gemm(const GemmLaunch& p, hipStream_t s) {
     float* xs = reinterpret_cast<float*>(xt + static_cast<size_t>(m_pad) * (p.cols / 4));
     float* ts = xs + static_cast<size_t>(m_pad) * (p.cols / 64);
     const int nk = p.cols / 2048;
-    const bool vec = prep_vec_ok(p) && (nk == 1 || nk == 2 || nk == 6) &&
-                     (nk == 1 ? launch_prep_vec<1>(p, m_pad, xt, xs, ts, s)
-                              : nk == 2 ? launch_prep_vec<2>(p, m_pad, xt, xs, ts, s)
-                                        : launch_prep_vec<6>(p, m_pad, xt, xs, ts, s));
-    if (!vec)
+    const int vec = prep_vec_ok(p) ? nk : 0;
+    if (vec == 1) launch_prep_vec<1>(p, m_pad, xt, xs, ts, s);
+    else if (vec == 2) launch_prep_vec<2>(p, m_pad, xt, xs, ts, s);
+    else if (vec == 3) launch_prep_vec<3>(p, m_pad, xt, xs, ts, s);
+    else if (vec == 4) launch_prep_vec<4>(p, m_pad, xt, xs, ts, s);
+    else if (vec == 6) launch_prep_vec<6>(p, m_pad, xt, xs, ts, s);
+    else
         hipLaunchKernelGGL(prep_x_kernel, dim3(m_pad), dim3(256), 0, s, p.x, p.ldx, p.m, p.cols, p.pro, p.ldz, xt, xs, ts);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     float* part = plan.splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(p.workspace) +
