@@ -321,7 +321,11 @@ static bool prep_vec_ok(const GemmLaunch& p) {
 // goes straight from memory into LDS, XS - 1 groups ahead for x (an LDS image in
 // operand order, read back one conflict-free KiB per fragment), two for the codes
 // (two groups of a row at a time) and a quad of groups for the scales; one
-// barrier per group.  A lane reads 16 bytes of codes per tile and group and
+// barrier per group, before the group's last step: the next group's first reads
+// and the transfers that reuse its LDS run under that step's MFMAs, one transfer
+// between two of them (with the barrier after the step and a group's transfers
+// requested together: 12352x4096, 512 tokens 103 us, now 99; 10240 rows 95, now
+// 90; 24576 rows 128 tokens 66, now 62.5).  A lane reads 16 bytes of codes per tile and group and
 // unpacks a word of 8 with one shift, four three-input bit ops and four packed
 // fp16 subtractions.  The LDS reads, the unpacking and the scaling of a finished
 // group's sums are placed between the MFMAs.
@@ -414,6 +418,11 @@ __device__ __forceinline__ u32x4 buf_words(const void* p, uint32_t bytes) {
                  static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(bytes)), kBufWord3};
 }
 
+template <typename V>
+__device__ __forceinline__ V lds_at(uint32_t byte) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) V*>(byte);
+}
+
 template <int WGR, int WGT, int TI, int TJ, int XS, int META>
 __global__ void __launch_bounds__(kWave * WGR * WGT) __attribute__((amdgpu_waves_per_eu(TI * TJ <= 2 ? 4 : 2)))
 gemm_w4_mfma_kernel(GemmArgs a) {
@@ -421,9 +430,7 @@ gemm_w4_mfma_kernel(GemmArgs a) {
     using T = GemmTile<WGR, WGT, TI, TJ, XS>;
     constexpr int BR = T::kBR, BT = T::kBT, XU = T::kXU, AU = T::kAU, SU = T::kSU, NT = T::kThreads;
     extern __shared__ u32x4 gemm_lds[];
-    u32x4* xl = gemm_lds;                                     // [XS stages][kXStage]
-    u32x4* al = xl + XS * T::kXStage;                          // [BR][8]
-    u32x4* sl = al + 8 * BR;  // [BR] metadata words of the quad's groups
+    // LDS: x [XS stages][kXStage], codes [BR][8], metadata words of the quad's groups [BR]
     // Tile of this block.  Blocks are dealt to the 8 XCDs round robin in
     // launch order; a weight slab (BR rows of one K split, a "unit") is read
     // by every token tile, so the token tiles of a unit are given launch
@@ -461,12 +468,9 @@ gemm_w4_mfma_kernel(GemmArgs a) {
     const uint32_t x_tile = static_cast<uint32_t>(t0 >> 5) * kXTile * 16u;
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
         reinterpret_cast<__attribute__((address_space(3))) uint8_t*>(reinterpret_cast<uintptr_t>(gemm_lds)))) ;
-    auto load_x = [&](int g, int st) {
-        const uint32_t so = static_cast<uint32_t>(g) * x_group + x_tile;
-        const uint32_t d = lds0 + (st * T::kXStage + wid * kWave) * 16u;
-#pragma unroll
-        for (int j = 0; j < XU; ++j)
-            buffer_to_lds16(x_r, static_cast<uint32_t>(tid) * 16u, so + NT * 16u * j, d + NT * 16u * j);
+    auto load_x = [&](int g, int st, int j) {
+        buffer_to_lds16(x_r, static_cast<uint32_t>(tid) * 16u, static_cast<uint32_t>(g) * x_group + x_tile + NT * 16u * j,
+                        lds0 + (st * T::kXStage + wid * kWave + NT * j) * 16u);
     };
 
     // codes, two groups (half a quad) at a time: LDS row r (64 bytes) of half-quad p holds in slot n the piece
@@ -477,28 +481,24 @@ gemm_w4_mfma_kernel(GemmArgs a) {
     const int apiece = (tid ^ (tid >> 4)) & 3;
     const uint32_t aoff = static_cast<uint32_t>(r0 + (tid >> 2)) * row_bytes + (apiece & 1) * 16u;
     // (the whole offset in the vector operand: the range check must see all of it)
-    auto load_a = [&](int g, int hq) {  // half-quad hq of the quad at g
+    auto load_a = [&](int g, int hq, int j) {  // half-quad hq of the quad at g
         const int c = g >> 6;
         const uint32_t half = static_cast<uint32_t>(c == lastc ? gc_last : 64) * 16u;
         const uint32_t off = aoff + (apiece & 2 ? half : 0u) + static_cast<uint32_t>(c) * 2048u + ((g & 63) + 2 * hq) * 16u;
-        const uint32_t d = lds0 + (XS * T::kXStage + hq * BR * 4 + wid * kWave) * 16u;
-#pragma unroll
-        for (int j = 0; j < AU; ++j) buffer_to_lds16(nib_r, off + (NT / 4) * j * row_bytes, 0, d + NT * 16u * j);
+        buffer_to_lds16(nib_r, off + (NT / 4) * j * row_bytes, 0,
+                        lds0 + (XS * T::kXStage + hq * BR * 4 + wid * kWave + NT * j) * 16u);
     };
     // scales: word i = tid + NT j is group i & 3 of the quad, row i >> 2
     const u32x4 meta_w = buf_words(a.meta, meta_total_bytes<META>(static_cast<uint32_t>(a.rows), static_cast<uint32_t>(G)));
     const uint32_t soff = (static_cast<uint32_t>(r0 + (tid >> 2)) * G + (tid & 3)) * kMetaBytes;
-    auto load_s = [&](int g) {
-        const uint32_t d = lds0 + (XS * T::kXStage + 8 * BR) * 16u + wid * kWave * 4u;
-#pragma unroll
-        for (int j = 0; j < SU; ++j)
-            buffer_to_lds<META == 2 ? 2 : 4>(meta_w, soff + static_cast<uint32_t>(g + (NT / 4) * j * G) * kMetaBytes, 0,
-                                             d + NT * 4u * j);
+    auto load_s = [&](int g, int j) {
+        buffer_to_lds<META == 2 ? 2 : 4>(meta_w, soff + static_cast<uint32_t>(g + (NT / 4) * j * G) * kMetaBytes, 0,
+                                         lds0 + (XS * T::kXStage + 8 * BR) * 16u + (wid * kWave + NT * j) * 4u);
     };
     // One MFMA step (16 of the group's 64 columns) multiplies every tile pair by x_hi and x_lo, in a fixed
     // order with the next step's LDS reads and unpacking between the MFMAs; a group's sums are scaled into the
-    // result at the next group's first step, tile by tile before the tile's sums start again from 0.
-    u32x4 cw[TI];       // the group's codes
+    // result from its last step to the next group's first, tile by tile before the tile's sums start again from 0.
+    u32x4 cw[2][TI];    // codes of the group and of the next
     u32x4 sq[TI];       // metadata words of the quad
     float sv[2][TI];    // scales of the group and of the one before
     half8 xf[2][TJ][2]; // x_hi, x_lo fragments of this step and the next
@@ -508,23 +508,28 @@ gemm_w4_mfma_kernel(GemmArgs a) {
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < TJ; ++j) acc[i][j] = t[i][j] = floatx16{};
-    const half8* xbase = reinterpret_cast<const half8*>(xl + wj * kXTile) + lane;
+    // LDS addresses of the lane, one register each (opaque: the compiler otherwise keeps one per read, hoisted out
+    // of the loop); everything else is a constant offset
+    uint32_t x16 = lds0 + (wj * kXTile + lane) * 16u;
+    const uint32_t arow = lds0 + XS * T::kXStage * 16u + (wr + lr) * 64u;
+    uint32_t a_even = arow + ((2 * lh) ^ ((lr >> 2) & 3)) * 16u, a_odd = arow + ((2 * lh + 1) ^ ((lr >> 2) & 3)) * 16u;
+    uint32_t s16 = lds0 + (XS * T::kXStage + 8 * BR + wr + lr) * 16u;
+    asm("" : "+v"(x16), "+v"(a_even), "+v"(a_odd), "+v"(s16));
     auto read_x = [&](int st, int s, int b) {
-        const half8* xp = xbase + st * T::kXStage + s * 64;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
-            xf[b][j][0] = xp[j * kXTile];
-            xf[b][j][1] = xp[j * kXTile + kXLo];
+            const uint32_t at = x16 + (st * T::kXStage + s * 64 + j * kXTile) * 16u;
+            xf[b][j][0] = lds_at<half8>(at);
+            xf[b][j][1] = lds_at<half8>(at + kXLo * 16u);
         }
     };
     auto read_codes = [&](int u) {
 #pragma unroll
-        for (int i = 0; i < TI; ++i)
-            cw[i] = al[((u >> 1) * BR + wr + 32 * i + lr) * 4 + ((2 * lh + (u & 1)) ^ ((lr >> 2) & 3))];
+        for (int i = 0; i < TI; ++i) cw[u & 1][i] = lds_at<u32x4>((u & 1 ? a_odd : a_even) + ((u >> 1) * BR + 32 * i) * 64u);
     };
     auto read_scales = [&] {
 #pragma unroll
-        for (int i = 0; i < TI; ++i) sq[i] = sl[wr + 32 * i + lr];
+        for (int i = 0; i < TI; ++i) sq[i] = lds_at<u32x4>(s16 + 512u * i);
     };
     auto set_scale = [&](int u, bool in) {  // groups past g1 get scale 0
 #pragma unroll
@@ -538,9 +543,9 @@ gemm_w4_mfma_kernel(GemmArgs a) {
 #pragma unroll
         for (int v = 4 * part; v < 4 * part + 4; ++v) acc[i][j][v] = fmaf(sv[b][i], t[i][j][v], acc[i][j][v]);
     };
-    auto unpack = [&](int b, int s, int n) {  // piece n of step s's unpacking: word n / 4
+    auto unpack = [&](int b, int p, int s, int n) {  // piece n of step s's unpacking: word n / 4
         const int i = n >> 2;
-        const uint32_t w = cw[i][s];
+        const uint32_t w = cw[p][i][s];
         switch (n & 3) {
             case 0: cf[b][i][0] = unpack_pair<0>(w); break;
             case 1: cf[b][i][1] = unpack_pair<1>(w); break;
@@ -558,38 +563,73 @@ gemm_w4_mfma_kernel(GemmArgs a) {
         return s0 < s1 ? s0 : s1;
     };
     static_assert(XS == 2 || XS == 4, "the stage of a group is a constant of its place in the quad");
-    load_s(g0);
-    load_a(g0, 0);
-    load_a(g0, 1);
 #pragma unroll
-    for (int e = 0; e < XS - 1; ++e) load_x(min(g0 + e, glast), e);
+    for (int j = 0; j < SU; ++j) load_s(g0, j);
+#pragma unroll
+    for (int j = 0; j < 2 * AU; ++j) load_a(g0, j / AU, j % AU);
+#pragma unroll
+    for (int e = 0; e < (XS - 1) * XU; ++e) load_x(min(g0 + e / XU, glast), e / XU, e % XU);
 #pragma unroll
     for (int i = 0; i < TI; ++i) sv[1][i] = 0.0f;
     wait_transfers<0>();
     __syncthreads();
+    // A group's phase runs from the barrier before its first reads to the next.  It requests the x that is XS - 1
+    // groups ahead (the stage was last read before the barrier), then the next quad's scales (u = 0) or half of its
+    // codes (u odd), whose LDS was last read before it too, at most one transfer before each MFMA.
+    auto request = [&](int g, int u, int slot) {  // slot: MFMAs of the phase before
+        const int gq = min((g & ~3) + 4, glast & ~3);
+#pragma unroll
+        for (int j = 0; j < XU; ++j)
+            if (slot == j) load_x(min(g + XS - 1, glast), (u + XS - 1) % XS, j);
+#pragma unroll
+        for (int j = 0; j < SU; ++j)
+            if (u == 0 && slot == XU + j) load_s(gq, j);
+#pragma unroll
+        for (int j = 0; j < AU; ++j)
+            if ((u & 1) && slot == XU + j) load_a(gq, u >> 1, j);
+    };
+    static_assert(XU + AU <= 4 * NM && XU + SU <= 4 * NM, "every request within the phase");
+    read_x(0, 0, 0);
     read_scales();
     read_codes(0);
+    __syncthreads();  // the first scales are read before the next are requested
 #pragma unroll
-    for (int n = 0; n < 4 * TI; ++n) unpack(0, 0, n);
+    for (int n = 0; n < NM; ++n) request(g0, 0, n);
+#pragma unroll
+    for (int n = 0; n < 4 * TI; ++n) unpack(0, 0, 0, n);
     for (int g = g0; g < g1; g += 4) {
-        const int gq = min(g + 4, glast & ~3);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {  // group g + u (past g1: scales 0), x stage u % XS
-            read_x(u % XS, 0, 0);
-            load_x(min(g + u + XS - 1, glast), (u + XS - 1) % XS);  // its stage was last read before the barrier
-            // the next quad: the scales, and a half-quad's last codes, were read before the barrier
-            if (u == 0) load_s(gq);
-            if (u & 1) load_a(gq, u >> 1);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int b = k & 1;
-                if (k < 3) read_x(u % XS, k + 1, b ^ 1);
-                else read_codes((u + 1) & 3);
+                if (k == 1) read_codes((u + 1) & 3);
                 if (k == 2) set_scale(u, g + u < g1);
-                if (k == 3 && u == 3) read_scales();
+                if (k == 2 && u == 3) read_scales();
+                if (k < 3) {
+                    read_x(u % XS, k + 1, b ^ 1);
+                } else {
+                    // All of the group's x is in registers: the barrier, and the next group's first reads under this
+                    // step's MFMAs.  Landed before it: the next group's x, the codes requested in the phase before
+                    // (each has had XS - 1 or two phases' time), the scales (three phases').
+                    if constexpr (XS == 2) {
+                        if (u == 0) wait_transfers<SU>();
+                        else if (u == 2) wait_transfers<0>();
+                        else wait_transfers<AU>();
+                    } else {
+                        if (u == 0) wait_transfers<XU + SU>();
+                        else if (u == 1) wait_transfers<2 * XU + SU + AU>();
+                        else if (u == 2) wait_transfers<XU>();
+                        else wait_transfers<2 * XU + AU>();
+                    }
+                    __syncthreads();
+                    read_x((u + 1) % XS, 0, b ^ 1);
+                }
 #pragma unroll
                 for (int n = 0; n < NM; ++n) {
                     const int pair = n >> 1, i = pair / TJ, j = pair % TJ;
+                    if (k == 3) request(g + u + 1, (u + 1) & 3, n);
+                    else request(g + u, u, NM * (k + 1) + n);
                     if (k == 3 || k == 0) {
 #pragma unroll
                         for (int q = 0; q < 4 * NP; ++q)
@@ -598,33 +638,19 @@ gemm_w4_mfma_kernel(GemmArgs a) {
                     if (k == 0 && (n & 1) == 0) t[i][j] = zero;
                     t[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[b][j][n & 1], __builtin_bit_cast(half8, cf[b][i]),
                                                                      t[i][j], 0, 0, 0);
-                    // the next step's codes: spread over this step's MFMAs, or over the second half of them where
-                    // the codes have just been requested
+                    // the next step's codes, spread over this step's MFMAs
 #pragma unroll
                     for (int q = 0; q < 4 * TI; ++q)
-                        if (k < 3 ? q * NM / (4 * TI) == n : NP + q * NP / (4 * TI) == n) unpack(b ^ 1, (k + 1) & 3, q);
+                        if (q * NM / (4 * TI) == n) unpack(b ^ 1, k == 3 ? (u + 1) & 1 : u & 1, (k + 1) & 3, q);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            // Landed before the barrier: the next group's x, the codes requested in the group before (each has had
-            // XS - 1 or two groups' time), the scales (three groups').  In issue order a group requests x, then
-            // scales (u = 0) or codes (u odd).
-            if constexpr (XS == 2) {
-                if (u == 0) wait_transfers<SU>();
-                else if (u == 2) wait_transfers<0>();
-                else wait_transfers<AU>();
-            } else {
-                if (u == 0) wait_transfers<XU + SU>();
-                else if (u == 1) wait_transfers<2 * XU + SU + AU>();
-                else if (u == 2) wait_transfers<XU>();
-                else wait_transfers<2 * XU + AU>();
-            }
-            __syncthreads();
         }
     }
 #pragma unroll
     for (int q = 0; q < 4 * NP; ++q)
         if (scale_slot(q >> 2, q & 3) >= NM) scale_in(q >> 2, q & 3, 1);
+    wait_transfers<0>();  // the last phase's requests, which nothing reads
 
     // c0 term: K = G, lane half h takes groups gb + 8 h + 0..7 of its token / row.  All loads of a step are
     // issued before any use; groups past g1 read out of range (zero), so c0 and xs are 0.
