@@ -378,7 +378,9 @@ __global__ void __launch_bounds__(256) linear_scan_wave_kernel(LinearScanLaunch 
 // 2. the chunked recurrence (scan_chunk_prep_kernel, scan_chunk_state_kernel,
 //    below): parallel over 64-token chunks except for one pass over the chunks
 //    per (value head, 16 columns).
-// Workspace: conv output [tokens][conv_dim], (beta, g) [tokens][lv_n][2], then
+// Workspace: conv output by head, [2 lk_n][tokens][lk_hd] and [lv_n][tokens][lv_hd]
+// (a block of the chunk kernels reads one head: with rows of all heads its reads
+// lie a row apart and meet in few memory channels), (beta, g) [lv_n][tokens][2], then
 // per (chunk, value head) the record T [64][64], Wq [64][64], gamma [64],
 // gamma_last / gamma [64].
 // ---------------------------------------------------------------------------
@@ -427,11 +429,12 @@ __global__ void __launch_bounds__(256) linear_conv_prefill_kernel(LinearScanLaun
     } else if (threadIdx.x == 0) {
         const int vh = hb - 2 * p.lk_n;
         const size_t row = static_cast<size_t>(t) * p.mixed_stride + vh;
-        float* aux = p.ws + static_cast<size_t>(p.tokens) * conv_dim + (static_cast<size_t>(t) * p.lv_n + vh) * 2;
+        float* aux = p.ws + static_cast<size_t>(p.tokens) * conv_dim + (static_cast<size_t>(vh) * p.tokens + t) * 2;
         aux[0] = sigmoid_dev(p.b[row]);
         aux[1] = -expf(p.a_log[vh]) * softplus_dev(p.a[row] + p.dt_bias[vh]);  // log of the decay
     }
-    if (ok) p.ws[static_cast<size_t>(t) * conv_dim + c] = y;
+    const size_t head = static_cast<size_t>(c - static_cast<int>(threadIdx.x)) * p.tokens;  // its first value
+    if (ok) p.ws[head + static_cast<size_t>(t) * width + threadIdx.x] = y;
 }
 
 // The same pass for 128-channel heads and a conv kernel of KS taps, one block
@@ -494,13 +497,13 @@ __global__ void __launch_bounds__(128) linear_conv_prefill_tg_kernel(LinearScanL
     } else if (threadIdx.x < TG && g0 + static_cast<int>(threadIdx.x) < p.tokens) {
         const int t = g0 + threadIdx.x, vh = hb - 2 * p.lk_n;
         const size_t row = static_cast<size_t>(t) * p.mixed_stride + vh;
-        float* aux = p.ws + static_cast<size_t>(p.tokens) * conv_dim + (static_cast<size_t>(t) * p.lv_n + vh) * 2;
+        float* aux = p.ws + static_cast<size_t>(p.tokens) * conv_dim + (static_cast<size_t>(vh) * p.tokens + t) * 2;
         aux[0] = sigmoid_dev(p.b[row]);
         aux[1] = -expf(p.a_log[vh]) * softplus_dev(p.a[row] + p.dt_bias[vh]);  // log of the decay
     }
 #pragma unroll
     for (int k = 0; k < TG; ++k)
-        if (g0 + k < p.tokens) p.ws[static_cast<size_t>(g0 + k) * conv_dim + c] = y[k];
+        if (g0 + k < p.tokens) p.ws[(static_cast<size_t>(hb) * p.tokens + g0 + k) * 128 + threadIdx.x] = y[k];
     // the history after the chunk: inputs of tokens tokens - H .. tokens - 1, slots
     // tokens - g0 + i of the group that holds the last token
     if (g0 <= p.tokens - 1 && p.tokens - 1 < g0 + TG) {
@@ -533,35 +536,35 @@ __global__ void __launch_bounds__(128) linear_conv_prefill_tg_kernel(LinearScanL
 // Wq_ij = exp(G_i - G_j) (q_i . k_j) (j <= i); scan_chunk_state_kernel, one block
 // per (value head, 16 value columns), walks the chunks in order with the state
 // slice in LDS and the products on v_mfma_f32_16x16x4_f32 (fp32 operands, fp32
-// accumulation).  Same mathematics as the per-token recurrence
+// accumulation).  The prep kernel is one block per CU as well (32 heads, 500
+// tokens: 256), a chain of short phases bound by LDS latency: 16.2 us, 20.2 with
+// the sums of the log decays and the block products read from LDS word by word.  Same mathematics as the per-token recurrence
 // (custom_model.cpp:1074-1096), a different fp32 summation order.
 constexpr int kChunk = kChunkTokens;  // tokens per chunk
 constexpr int kChLd = 132;   // floats per 128-dim row in LDS (16-byte aligned rows)
 constexpr int kChLdT = 68;   // floats per 64-wide row in LDS
+constexpr int kChLdM = 20;   // floats per row of a 16 x 16 block in LDS
 constexpr int kChRec = kChunkRecord;  // floats per (value head, chunk) record
 
 static size_t scan_chunk_prep_lds() {
-    return sizeof(float) * (2 * static_cast<size_t>(kChunk) * kChLd + 2 * kChunk * kChLdT + 4 * 16 * 17 + 3 * kChunk);
+    return sizeof(float) * (2 * static_cast<size_t>(kChunk) * kChLd + 2 * kChunk * kChLdT + 4 * 16 * kChLdM + 3 * kChunk);
 }
 static size_t scan_chunk_state_lds() {
-    return sizeof(float) * (2 * static_cast<size_t>(kChunk) * kChLd + 2 * kChunk * kChLdT + 2 * 16 * kChLdT +
-                            16 * kChLd + kChunk * 16 + 3 * kChunk);
+    return sizeof(float) * (128 * kChLdT + 2 * 16 * kChLdT + 16 * kChLd);
 }
 
 // q and k rows of key head kh for the chunk's tokens [t0, t0 + n) -> LDS rows of
 // kChLd floats (rows past n are 0)
-__device__ __forceinline__ void stage_qk_rows(const LinearScanLaunch& p, int conv_dim, int kh, int t0, int n,
-                                              float* Ks, float* Qs) {
-    const __amdgpu_buffer_rsrc_t r = buf_rsrc(p.ws + static_cast<size_t>(t0) * conv_dim,
-                                              static_cast<uint32_t>(max(0, n)) * conv_dim * 4u);
-    const uint32_t kc = static_cast<uint32_t>(p.lk_n * 128 + kh * 128), qc = static_cast<uint32_t>(kh * 128);
+__device__ __forceinline__ void stage_qk_rows(const LinearScanLaunch& p, int kh, int t0, int n, float* Ks, float* Qs) {
+    const uint32_t bytes = static_cast<uint32_t>(max(0, n)) * 512u;
+    const __amdgpu_buffer_rsrc_t rq = buf_rsrc(p.ws + (static_cast<size_t>(kh) * p.tokens + t0) * 128, bytes);
+    const __amdgpu_buffer_rsrc_t rk = buf_rsrc(p.ws + (static_cast<size_t>(p.lk_n + kh) * p.tokens + t0) * 128, bytes);
     u32x4 kv[8], qv[8];  // all loads in flight before the first store
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-        const int e = static_cast<int>(threadIdx.x) + 256 * u, row = e >> 5, d4 = e & 31;
-        const uint32_t base = static_cast<uint32_t>(row) * conv_dim + 4u * d4;
-        kv[u] = __builtin_amdgcn_raw_buffer_load_b128(r, (base + kc) * 4u, 0, 0);
-        qv[u] = __builtin_amdgcn_raw_buffer_load_b128(r, (base + qc) * 4u, 0, 0);
+        const uint32_t at = (threadIdx.x + 256u * u) * 16u;
+        kv[u] = __builtin_amdgcn_raw_buffer_load_b128(rk, at, 0, 0);
+        qv[u] = __builtin_amdgcn_raw_buffer_load_b128(rq, at, 0, 0);
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -577,8 +580,8 @@ __global__ void __launch_bounds__(256) scan_chunk_prep_kernel(LinearScanLaunch p
     float* Qs = Ks + kChunk * kChLd;                 // [64][kChLd]
     float* Am = Qs + kChunk * kChLd;                 // [64][kChLdT] A (strictly lower)
     float* Tm = Am + kChunk * kChLdT;                // [64][kChLdT] T = (I + A)^{-1}, by 16 x 16 blocks
-    float* Mw = Tm + kChunk * kChLdT;                // [4 waves][16][17] block products
-    float* Gc = Mw + 4 * 16 * 17;                    // [64] cumulative log decay
+    float* Mw = Tm + kChunk * kChLdT;                // [4 waves][16][kChLdM] block products
+    float* Gc = Mw + 4 * 16 * kChLdM;                   // [64] cumulative log decay
     float* Bt = Gc + kChunk;                         // [64] beta
     float* gl = Bt + kChunk;                         // [64] log decay
     const int vh = blockIdx.x, ch = blockIdx.y, t0 = ch * kChunk;
@@ -587,17 +590,24 @@ __global__ void __launch_bounds__(256) scan_chunk_prep_kernel(LinearScanLaunch p
     const int kh = __builtin_amdgcn_readfirstlane(min(p.lk_n - 1, vh / factor));
     const int conv_dim = 2 * p.lk_n * 128 + p.lv_n * p.lv_hd;
     const int tid = threadIdx.x;
-    stage_qk_rows(p, conv_dim, kh, t0, n, Ks, Qs);
+    stage_qk_rows(p, kh, t0, n, Ks, Qs);
     if (tid < kChunk) {  // tokens past n: beta 0, log decay 0 (the state passes unchanged)
         const float* aux = p.ws + static_cast<size_t>(p.tokens) * conv_dim;
-        const size_t ai = (static_cast<size_t>(t0 + tid) * p.lv_n + vh) * 2;
+        const size_t ai = (static_cast<size_t>(vh) * p.tokens + t0 + tid) * 2;
         Bt[tid] = tid < n ? aux[ai] : 0.0f;
         gl[tid] = tid < n ? aux[ai + 1] : 0.0f;
     }
     __syncthreads();
     if (tid < kChunk) {
+        float4 g[kChunk / 4];  // every load before the chain of additions
+#pragma unroll
+        for (int l = 0; l < kChunk / 4; ++l) g[l] = *reinterpret_cast<const float4*>(gl + 4 * l);
         float acc = 0.0f;
-        for (int l = 0; l <= tid; ++l) acc += gl[l];
+#pragma unroll
+        for (int l = 0; l < kChunk; ++l) {
+            const float4 v = g[l >> 2];
+            acc += l <= tid ? ((l & 3) == 0 ? v.x : (l & 3) == 1 ? v.y : (l & 3) == 2 ? v.z : v.w) : 0.0f;
+        }
         Gc[tid] = acc;
     }
     // K K^T and Q K^T on v_mfma_f32_16x16x4_f32: wave w takes rows 16 w .. 16 w + 15
@@ -672,35 +682,44 @@ __global__ void __launch_bounds__(256) scan_chunk_prep_kernel(LinearScanLaunch p
         const int bi = w + dist, bj = w;
         const bool task = bi < 4;
         float m4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        // d += row (16 values) times the 4 columns at col (rows ld apart); every LDS read before the products
+        auto madd = [](const float* row, const float* col, int ld, float (&d)[4]) {
+            float4 a[4], t[16];
+#pragma unroll
+            for (int mm = 0; mm < 4; ++mm) a[mm] = *reinterpret_cast<const float4*>(row + 4 * mm);
+#pragma unroll
+            for (int mm = 0; mm < 16; ++mm) t[mm] = *reinterpret_cast<const float4*>(col + mm * ld);
+#pragma unroll
+            for (int mm = 0; mm < 16; ++mm) {
+                const float4 q = a[mm >> 2];
+                const float f = (mm & 3) == 0 ? q.x : (mm & 3) == 1 ? q.y : (mm & 3) == 2 ? q.z : q.w;
+                d[0] += f * t[mm].x;
+                d[1] += f * t[mm].y;
+                d[2] += f * t[mm].z;
+                d[3] += f * t[mm].w;
+            }
+        };
         if (task)
             for (int k = bj; k < bi; ++k)
-#pragma unroll
-                for (int mm = 0; mm < 16; ++mm) {
-                    const float a = Am[(16 * bi + br) * kChLdT + 16 * k + mm];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) m4[e] += a * Tm[(16 * k + mm) * kChLdT + 16 * bj + bc + e];
-                }
-        float* mw = Mw + w * 16 * 17;
-        if (task)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) mw[br * 17 + bc + e] = m4[e];
+                madd(Am + (16 * bi + br) * kChLdT + 16 * k, Tm + 16 * k * kChLdT + 16 * bj + bc, kChLdT, m4);
+        float* mw = Mw + w * 16 * kChLdM;
+        if (task) *reinterpret_cast<float4*>(mw + br * kChLdM + bc) = make_float4(m4[0], m4[1], m4[2], m4[3]);
         __syncthreads();
         if (task) {
             float t4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int mm = 0; mm < 16; ++mm) {
-                const float d = Tm[(16 * bi + br) * kChLdT + 16 * bi + mm];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) t4[e] += d * mw[mm * 17 + bc + e];
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Tm[(16 * bi + br) * kChLdT + 16 * bj + bc + e] = -t4[e];
+            madd(Tm + (16 * bi + br) * kChLdT + 16 * bi, mw + bc, kChLdM, t4);
+            *reinterpret_cast<float4*>(Tm + (16 * bi + br) * kChLdT + 16 * bj + bc) =
+                make_float4(-t4[0], -t4[1], -t4[2], -t4[3]);
         }
         __syncthreads();
     }
-    for (int e = tid; e < kChunk * kChunk; e += 256) {
-        const int i = e >> 6, j = e & 63;
-        rec[e] = (j >> 4) <= (i >> 4) ? Tm[i * kChLdT + j] : 0.0f;  // blocks above the diagonal are 0
+    // buffer stores: a record need only be aligned to 4 bytes
+    const __amdgpu_buffer_rsrc_t rec_r = buf_rsrc(rec, kChRec * 4u);
+    for (int e = tid; e < kChunk * kChunk / 4; e += 256) {
+        const int i = e >> 4, j = 4 * (e & 15);
+        u32x4 v = *reinterpret_cast<const u32x4*>(Tm + i * kChLdT + j);
+        if ((j >> 4) > (i >> 4)) v = u32x4{0u, 0u, 0u, 0u};  // blocks above the diagonal are 0
+        __builtin_amdgcn_raw_buffer_store_b128(v, rec_r, e * 16u, 0, 0);
     }
     if (tid < kChunk) {
         rec[2 * kChunk * kChunk + tid] = expf(Gc[tid]);                          // gamma_i
@@ -708,220 +727,214 @@ __global__ void __launch_bounds__(256) scan_chunk_prep_kernel(LinearScanLaunch p
     }
 }
 
-// a chunk's inputs in registers: q / k rows, T, Wq, the value slice, beta and
-// the decay factors (loaded for chunk c + 1 while chunk c is computed)
-struct ChunkRegs {
-    u32x4 k[8], q[8], t[4], wq[4];
-    float v[4], bet, gam, del;
-};
-
-__global__ void __launch_bounds__(256) scan_chunk_state_kernel(LinearScanLaunch p) {
+// Eight waves.  Wave w < 4 computes X = K S_0, R and U for tokens 16 w .. 16 w + 15, wave w + 4 computes
+// Y = Q S_0 and the output for the same tokens, and wave w updates state rows 16 w .. 16 w + 15; the output of a chunk
+// is computed under the next chunk's X, Y under U, so that each SIMD has two waves with products to issue.  What
+// only a wave's own products read (its rows of K and T or Q and Wq, its values and gates) goes from memory straight
+// into the lanes that feed the MFMAs, requested for the next chunk as soon as this chunk has used it.  LDS carries
+// what crosses waves: K^T (for the state update), R and U (transposed: a lane's operand is a contiguous run) and
+// the state slice.
+// What bounds it: one block per CU (32 heads of 128 columns: 256 blocks), so a chunk is 128 fp32 MFMAs per SIMD (32
+// clocks each, 1.7 us) and three barriers between dependent products.  32 heads, 500 tokens: 34.7 us (30 without the loads); four
+// waves with every operand staged through LDS (five barriers, 290 KB of LDS traffic a chunk) 41.8, four waves with
+// the operands straight into registers 39.4.
+constexpr int kStateThreads = 512;
+__global__ void __launch_bounds__(kStateThreads) scan_chunk_state_kernel(LinearScanLaunch p) {
     extern __shared__ float4 scan_lds[];
-    float* Kc = reinterpret_cast<float*>(scan_lds);  // [64][kChLd]
-    float* Qc = Kc + kChunk * kChLd;                 // [64][kChLd]
-    float* Tc = Qc + kChunk * kChLd;                 // [64][kChLdT]
-    float* Wc = Tc + kChunk * kChLdT;                // [64][kChLdT]
-    // R, U and the state slice are kept transposed (column-major in the value
-    // column): the MFMA operand a lane needs is then a contiguous run
-    float* Rt = Wc + kChunk * kChLdT;                // [16][kChLdT] R^T
+    float* Kt = reinterpret_cast<float*>(scan_lds);  // [128][kChLdT] K^T
+    float* Rt = Kt + 128 * kChLdT;                   // [16][kChLdT] R^T
     float* Ut = Rt + 16 * kChLdT;                    // [16][kChLdT] U^T
     float* St = Ut + 16 * kChLdT;                    // [16][kChLd] the state slice, transposed
-    float* Vc = St + 16 * kChLd;                     // [64][16]
-    float* gam = Vc + kChunk * 16;                   // [64]
-    float* del = gam + kChunk;                       // [64]
-    float* bet = del + kChunk;                       // [64]
     const int vh = blockIdx.x, j0 = blockIdx.y * 16;
     const int factor = max(1, p.lv_n / max(1, p.lk_n));
     const int kh = __builtin_amdgcn_readfirstlane(min(p.lk_n - 1, vh / factor));
     const int dv = p.lv_hd;
     const int conv_dim = 2 * p.lk_n * 128 + p.lv_n * dv;
     const int chunks = __builtin_amdgcn_readfirstlane((p.tokens + kChunk - 1) / kChunk);
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const bool outputs = w >= 4;
+    const int wt = w & 3;
     const int li = lane & 15, lq = lane >> 4;  // MFMA operand row / column li, k slot lq
     const bool cact = j0 + li < dv;
     const float rdk = 1.0f / sqrtf(128.0f);
     float* S = p.state + static_cast<size_t>(vh) * 128 * dv;
     const float* aux = p.ws + static_cast<size_t>(p.tokens) * conv_dim;
     const float* recs = aux + static_cast<size_t>(p.tokens) * p.lv_n * 2;
-    const uint32_t kcol = static_cast<uint32_t>(p.lk_n * 128 + kh * 128), qcol = static_cast<uint32_t>(kh * 128);
-    const uint32_t vcol = static_cast<uint32_t>(2 * p.lk_n * 128 + vh * dv + j0);
-    // every load is a range-checked buffer load issued back to back: tokens past
-    // the prompt and chunks past the last read 0
-    // (sizes and bases through readfirstlane: scalar buffer descriptors)
-    auto load_chunk = [&](int ch, ChunkRegs& r) {
+    // byte offsets of the lane's operands: every load is a range-checked buffer load, tokens past the prompt and
+    // chunks past the last read 0 (sizes and bases through readfirstlane: scalar buffer descriptors).  The
+    // contraction index of every product is a permutation shared by both operands: at step 4 u + e, k slot lq takes
+    // dim or token 16 u + 4 lq + e, so an operand is 16 contiguous bytes per u and four lanes read 64.
+    const uint32_t xoff = static_cast<uint32_t>(16 * wt + li) * 512u + 16u * lq;  // q or k row
+    const uint32_t moff = static_cast<uint32_t>(16 * wt + li) * (kChunk * 4u) + 16u * lq +
+                          (outputs ? kChunk * kChunk * 4u : 0u);  // Wq or T row
+    const uint32_t voff = cact ? static_cast<uint32_t>((16 * wt + 4 * lq) * dv + j0 + li) * 4u : kBufOOB;
+    const uint32_t boff = static_cast<uint32_t>(16 * wt + 4 * lq) * 8u;
+    const uint32_t goff = 2u * kChunk * kChunk * 4u;  // gamma, then gamma_last / gamma
+    const float* xhead = p.ws + static_cast<size_t>(outputs ? kh : p.lk_n + kh) * p.tokens * 128;
+    const float* vhead = p.ws + (static_cast<size_t>(2 * p.lk_n) * 128 + static_cast<size_t>(vh) * dv) * p.tokens;
+    struct Rows { __amdgpu_buffer_rsrc_t x, v, rec, aux; };
+    auto rows = [&](int ch) {
         const int t0 = __builtin_amdgcn_readfirstlane(min(ch * kChunk, p.tokens));
         const int n = __builtin_amdgcn_readfirstlane(max(0, min(kChunk, p.tokens - t0)));
         const int cr = __builtin_amdgcn_readfirstlane(min(ch, chunks - 1));
-        const uint32_t rbytes = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(ch < chunks ? kChRec * 4 : 0));
-        const __amdgpu_buffer_rsrc_t rc =
-            buf_rsrc(p.ws + static_cast<size_t>(t0) * conv_dim, static_cast<uint32_t>(n) * conv_dim * 4u);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int e = tid + 256 * u, row = e >> 5, d4 = e & 31;
-            const uint32_t base = static_cast<uint32_t>(row) * conv_dim + 4u * d4;
-            r.k[u] = __builtin_amdgcn_raw_buffer_load_b128(rc, (base + kcol) * 4u, 0, 0);
-            r.q[u] = __builtin_amdgcn_raw_buffer_load_b128(rc, (base + qcol) * 4u, 0, 0);
-        }
-        const __amdgpu_buffer_rsrc_t rr = buf_rsrc(recs + static_cast<size_t>(cr * p.lv_n + vh) * kChRec, rbytes);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t e4 = static_cast<uint32_t>(tid + 256 * u);
-            r.t[u] = __builtin_amdgcn_raw_buffer_load_b128(rr, e4 * 16u, 0, 0);
-            r.wq[u] = __builtin_amdgcn_raw_buffer_load_b128(rr, kChunk * kChunk * 4u + e4 * 16u, 0, 0);
-        }
-        const int vi = tid >> 2, vc = 4 * (tid & 3);  // value rows x 4 columns
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            r.v[e] = buf_load_f32(rc, j0 + vc + e < dv ? (static_cast<uint32_t>(vi) * conv_dim + vcol + vc + e) * 4u : kBufOOB);
-        const __amdgpu_buffer_rsrc_t ra =
-            buf_rsrc(aux + static_cast<size_t>(t0) * p.lv_n * 2, static_cast<uint32_t>(n) * p.lv_n * 8u);
-        r.bet = buf_load_f32(ra, tid < kChunk ? (static_cast<uint32_t>(tid) * p.lv_n * 2 + vh * 2) * 4u : kBufOOB);
-        r.gam = buf_load_f32(rr, tid < kChunk ? (2 * kChunk * kChunk + tid) * 4u : kBufOOB);
-        r.del = buf_load_f32(rr, tid < kChunk ? (2 * kChunk * kChunk + kChunk + tid) * 4u : kBufOOB);
+        return Rows{buf_rsrc(xhead + static_cast<size_t>(t0) * 128, static_cast<uint32_t>(n) * 512u),
+                    buf_rsrc(vhead + static_cast<size_t>(t0) * dv, static_cast<uint32_t>(n) * dv * 4u),
+                    buf_rsrc(recs + static_cast<size_t>(cr * p.lv_n + vh) * kChRec,
+                             static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(ch < chunks ? kChRec * 4 : 0))),
+                    buf_rsrc(aux + (static_cast<size_t>(vh) * p.tokens + t0) * 2, static_cast<uint32_t>(n) * 8u)};
     };
-    auto store_chunk = [&](const ChunkRegs& r) {
+    auto load4 = [](__amdgpu_buffer_rsrc_t r, uint32_t off, float* d) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int e = tid + 256 * u, row = e >> 5, d4 = e & 31;
-            *reinterpret_cast<u32x4*>(Kc + row * kChLd + 4 * d4) = r.k[u];
-            *reinterpret_cast<u32x4*>(Qc + row * kChLd + 4 * d4) = r.q[u];
-        }
+        for (int e = 0; e < 4; ++e) d[e] = __uint_as_float(v[e]);
+    };
+    float x[32], mt[16], v4[4], bet[4], gam[4], dl[16], glast;  // x: K or Q rows, mt: T or Wq rows
+    auto load_x = [&](const Rows& r) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e4 = tid + 256 * u, i = e4 >> 4, j4 = e4 & 15;
-            *reinterpret_cast<u32x4*>(Tc + i * kChLdT + 4 * j4) = r.t[u];
-            *reinterpret_cast<u32x4*>(Wc + i * kChLdT + 4 * j4) = r.wq[u];
-        }
+        for (int u = 0; u < 8; ++u) load4(r.x, xoff + 64u * u, x + 4 * u);
+    };
+    auto load_m = [&](const Rows& r) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) Vc[(tid >> 2) * 16 + 4 * (tid & 3) + e] = r.v[e];
-        if (tid < kChunk) {
-            bet[tid] = r.bet;
-            gam[tid] = r.gam;
-            del[tid] = r.del;
+        for (int u = 0; u < 4; ++u) load4(r.rec, moff + 64u * u, mt + 4 * u);
+    };
+    auto load_values = [&](const Rows& r) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            v4[v] = buf_load_f32(r.v, voff + static_cast<uint32_t>(v) * dv * 4u);
+            bet[v] = buf_load_f32(r.aux, boff + 8u * v);
         }
     };
-    for (int e = tid; e < 128 * 16; e += 256) {
+    auto load_gamma = [&](const Rows& r) { load4(r.rec, goff + (16 * wt + 4 * lq) * 4u, gam); };
+    auto load_decay = [&](const Rows& r) {
+        glast = buf_load_f32(r.rec, goff + (kChunk - 1) * 4u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load4(r.rec, goff + (kChunk + 16 * u + 4 * lq) * 4u, dl + 4 * u);
+    };
+    // a float4 of LDS into four registers
+    auto ld4 = [](const float* a, float* d) {
+        const float4 v = *reinterpret_cast<const float4*>(a);
+        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+    };
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto times_state = [&] {  // x S_0, two chains (even and odd steps)
+        float sp[32];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ld4(St + li * kChLd + 16 * u + 4 * lq, sp + 4 * u);
+        floatx4 r0 = zero4, r1 = zero4;
+#pragma unroll
+        for (int st = 0; st < 32; st += 2) {
+            r0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[st], sp[st], r0, 0, 0, 0);
+            r1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[st + 1], sp[st + 1], r1, 0, 0, 0);
+        }
+        return r0 + r1;
+    };
+    auto times_rows = [&](const float (&b)[16]) {  // mt b
+        floatx4 r0 = zero4, r1 = zero4;
+#pragma unroll
+        for (int st = 0; st < 16; st += 2) {
+            r0 = __builtin_amdgcn_mfma_f32_16x16x4f32(mt[st], b[st], r0, 0, 0, 0);
+            r1 = __builtin_amdgcn_mfma_f32_16x16x4f32(mt[st + 1], b[st + 1], r1, 0, 0, 0);
+        }
+        return r0 + r1;
+    };
+    floatx4 Y = zero4;
+    float ub[16];
+    auto output = [&](int ch) {  // O = diag(gamma) Y + Wq U of chunk ch
+        const floatx4 O = times_rows(ub);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = ch * kChunk + 16 * wt + 4 * lq + v;
+            if (t < p.tokens && cact)
+                p.out[static_cast<size_t>(t) * p.out_stride + static_cast<size_t>(vh) * dv + j0 + li] =
+                    (gam[v] * Y[v] + O[v]) * rdk;
+        }
+    };
+    {
+        const Rows r = rows(0);
+        load_x(r);
+        if (!outputs) {
+            load_values(r);
+            load_gamma(r);
+            load_m(r);
+        }
+        load_decay(r);
+    }
+    for (int e = tid; e < 128 * 16; e += kStateThreads) {
         const int d = e >> 4, cc = e & 15;
         St[cc * kChLd + d] = j0 + cc < dv ? S[static_cast<size_t>(d) * dv + j0 + cc] : 0.0f;
     }
-    // a float4 of LDS into four registers
-    auto ld4 = [](const float* q, float* d) {
-        const float4 v = *reinterpret_cast<const float4*>(q);
-        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
-    };
-    ChunkRegs nx;
-    load_chunk(0, nx);
-    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int ch = 0; ch < chunks; ++ch) {  // block-uniform
-        const int t0 = ch * kChunk, n = min(kChunk, p.tokens - t0);
-        __syncthreads();  // the previous chunk's LDS data have been read
-        store_chunk(nx);
+    __syncthreads();
+    // S_C = gamma_last S_0 + K^T diag(del) U: the wave's state rows.  The second and third barrier of a chunk.
+    auto update_state = [&](const Rows& nx) {
+        float kt[16], s4[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ld4(Kt + (16 * w + li) * kChLdT + 16 * u + 4 * lq, kt + 4 * u);
+        ld4(St + li * kChLd + 16 * w + 4 * lq, s4);
         __syncthreads();
-        load_chunk(ch + 1, nx);  // in flight during this chunk's products
-        // The contraction index of every product below is a permutation shared by
-        // both operands: lane (li, lq) feeds dims 32 lq + s (K S, Q S) or tokens
-        // 16 lq + s (T R, Wq U, K^T U) at step s, so its operands are contiguous.
-        // X = K S_0, Y = Q S_0 for the wave's 16 tokens
-        floatx4 X = zero4, Y = zero4;
-        {
-            float ka[32], qa[32], sp[32];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                ld4(Kc + (16 * w + li) * kChLd + 32 * lq + 4 * u, ka + 4 * u);
-                ld4(Qc + (16 * w + li) * kChLd + 32 * lq + 4 * u, qa + 4 * u);
-                ld4(St + li * kChLd + 32 * lq + 4 * u, sp + 4 * u);
-            }
-            floatx4 X1 = zero4, Y1 = zero4;  // two chains each (even / odd steps)
+        for (int u = 0; u < 4; ++u) ld4(Ut + li * kChLdT + 16 * u + 4 * lq, ub + 4 * u);
+        __builtin_amdgcn_sched_barrier(0);
+        floatx4 Sn, S1 = zero4;
 #pragma unroll
-            for (int st = 0; st < 32; st += 2) {
-                X = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[st], sp[st], X, 0, 0, 0);
-                Y = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[st], sp[st], Y, 0, 0, 0);
-                X1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[st + 1], sp[st + 1], X1, 0, 0, 0);
-                Y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[st + 1], sp[st + 1], Y1, 0, 0, 0);
-            }
-            X += X1;
-            Y += Y1;
+        for (int v = 0; v < 4; ++v) Sn[v] = glast * s4[v];
+#pragma unroll
+        for (int st = 0; st < 16; st += 2) {
+            Sn = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[st], ub[st] * dl[st], Sn, 0, 0, 0);
+            S1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[st + 1], ub[st + 1] * dl[st + 1], S1, 0, 0, 0);
         }
-        // R_i = b_i (v_i - gamma_i X_i) (rows 16 w + 4 lq + v, column li), stored transposed
-        {
+        Sn += S1;
+        *reinterpret_cast<float4*>(St + li * kChLd + 16 * w + 4 * lq) = make_float4(Sn[0], Sn[1], Sn[2], Sn[3]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_decay(nx);
+        __syncthreads();  // the new state is whole; K^T, R and U have been read
+    };
+    // The two kinds of wave run loops of their own with the same three barriers per chunk (a loop with branches kept
+    // the loads of both alive in copies, and waited for them there).  Loads for the next chunk overwrite registers
+    // behind their last use: the scheduling barriers keep them from being moved above it, which would need copies too.
+    if (outputs) {  // wave-uniform
+        for (int ch = 0; ch < chunks; ++ch) {
+            if (ch > 0) output(ch - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const Rows cur = rows(ch), nx = rows(ch + 1);
+            load_m(cur);
+            load_gamma(cur);
+            __syncthreads();
+            Y = times_state();
+            __builtin_amdgcn_sched_barrier(0);
+            load_x(nx);
+            update_state(nx);
+        }
+        output(chunks - 1);
+    } else {
+        for (int ch = 0; ch < chunks; ++ch) {
+            const Rows nx = rows(ch + 1);
+            __builtin_amdgcn_s_setprio(1);  // the chain that everything waits for
+            // R_i = b_i (v_i - gamma_i X_i) (rows 16 wt + 4 lq + v, column li), stored transposed; K^T
+            const floatx4 X = times_state();
+#pragma unroll
+            for (int st = 0; st < 32; ++st) Kt[(16 * (st >> 2) + 4 * lq + (st & 3)) * kChLdT + 16 * wt + li] = x[st];
             float r4[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = 16 * w + 4 * lq + v;
-                r4[v] = bet[i] * (Vc[i * 16 + li] - gam[i] * X[v]);
-            }
-            *reinterpret_cast<float4*>(Rt + li * kChLdT + 16 * w + 4 * lq) = make_float4(r4[0], r4[1], r4[2], r4[3]);
+            for (int v = 0; v < 4; ++v) r4[v] = bet[v] * (v4[v] - gam[v] * X[v]);
+            *reinterpret_cast<float4*>(Rt + li * kChLdT + 16 * wt + 4 * lq) = make_float4(r4[0], r4[1], r4[2], r4[3]);
+            __builtin_amdgcn_sched_barrier(0);
+            load_x(nx);
+            load_values(nx);
+            load_gamma(nx);
+            __syncthreads();
+            float rb[16];  // U = T R
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ld4(Rt + li * kChLdT + 16 * u + 4 * lq, rb + 4 * u);
+            __builtin_amdgcn_sched_barrier(0);
+            const floatx4 U = times_rows(rb);
+            *reinterpret_cast<float4*>(Ut + li * kChLdT + 16 * wt + 4 * lq) = make_float4(U[0], U[1], U[2], U[3]);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            load_m(nx);
+            update_state(nx);
         }
-        __syncthreads();
-        // U = T R for the wave's 16 tokens
-        floatx4 U = zero4;
-        {
-            float ta[16], rb[16];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                ld4(Tc + (16 * w + li) * kChLdT + 16 * lq + 4 * u, ta + 4 * u);
-                ld4(Rt + li * kChLdT + 16 * lq + 4 * u, rb + 4 * u);
-            }
-            floatx4 U1 = zero4;
-#pragma unroll
-            for (int st = 0; st < 16; st += 2) {
-                U = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[st], rb[st], U, 0, 0, 0);
-                U1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[st + 1], rb[st + 1], U1, 0, 0, 0);
-            }
-            U += U1;
-        }
-        *reinterpret_cast<float4*>(Ut + li * kChLdT + 16 * w + 4 * lq) = make_float4(U[0], U[1], U[2], U[3]);
-        __syncthreads();
-        // O = diag(gamma) Y + Wq U; the state update's U operand, scaled by del
-        floatx4 O = zero4;
-        float ub[16];
-        {
-            float wa[16], dl[16];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                ld4(Wc + (16 * w + li) * kChLdT + 16 * lq + 4 * u, wa + 4 * u);
-                ld4(Ut + li * kChLdT + 16 * lq + 4 * u, ub + 4 * u);
-                ld4(del + 16 * lq + 4 * u, dl + 4 * u);
-            }
-            floatx4 O1 = zero4;
-#pragma unroll
-            for (int st = 0; st < 16; st += 2) {
-                O = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[st], ub[st], O, 0, 0, 0);
-                O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[st + 1], ub[st + 1], O1, 0, 0, 0);
-            }
-            O += O1;
-#pragma unroll
-            for (int st = 0; st < 16; ++st) ub[st] *= dl[st];
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int i = 16 * w + 4 * lq + v;
-            if (i < n && cact)
-                p.out[static_cast<size_t>(t0 + i) * p.out_stride + static_cast<size_t>(vh) * dv + j0 + li] =
-                    (gam[i] * Y[v] + O[v]) * rdk;
-        }
-        // S_C = gamma_last S_0 + K^T diag(del) U: the wave's state rows 32 w .. 32 w + 31
-        floatx4 Sn[2];
-#pragma unroll
-        for (int rr = 0; rr < 2; ++rr) {
-            const int rt = 2 * w + rr;
-            float s4[4], kt[16];
-            ld4(St + li * kChLd + 16 * rt + 4 * lq, s4);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Sn[rr][v] = gam[kChunk - 1] * s4[v];
-#pragma unroll
-            for (int st = 0; st < 16; ++st) kt[st] = Kc[(16 * lq + st) * kChLd + 16 * rt + li];
-#pragma unroll
-            for (int st = 0; st < 16; ++st) Sn[rr] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[st], ub[st], Sn[rr], 0, 0, 0);
-        }
-        __syncthreads();  // every wave has read the old state
-#pragma unroll
-        for (int rr = 0; rr < 2; ++rr)
-            *reinterpret_cast<float4*>(St + li * kChLd + 16 * (2 * w + rr) + 4 * lq) =
-                make_float4(Sn[rr][0], Sn[rr][1], Sn[rr][2], Sn[rr][3]);
     }
-    __syncthreads();
-    for (int e = tid; e < 128 * 16; e += 256) {
+    for (int e = tid; e < 128 * 16; e += kStateThreads) {
         const int d = e >> 4, cc = e & 15;
         if (j0 + cc < dv) S[static_cast<size_t>(d) * dv + j0 + cc] = St[cc * kChLd + d];
     }
@@ -960,7 +973,8 @@ hipError_t launch_linear_scan(const LinearScanLaunch& p, hipStream_t s) {
         const int chunks = (p.tokens + kChunk - 1) / kChunk;
         hipLaunchKernelGGL(scan_chunk_prep_kernel, dim3(p.lv_n, chunks), dim3(256), scan_chunk_prep_lds(), s, p);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        hipLaunchKernelGGL(scan_chunk_state_kernel, dim3(p.lv_n, (p.lv_hd + 15) / 16), dim3(256), scan_chunk_state_lds(),
+        hipLaunchKernelGGL(scan_chunk_state_kernel, dim3(p.lv_n, (p.lv_hd + 15) / 16), dim3(kStateThreads),
+                           scan_chunk_state_lds(),
                            s, p);
         return hipGetLastError();
     }
