@@ -386,8 +386,11 @@ __device__ __forceinline__ uint32_t unpack_pair(uint32_t w) {
 // 16 bytes per lane from a buffer straight into LDS, lane l to byte lds + 16 l (lds wave-uniform).  Written as asm
 // because the compiler makes every LDS read after the builtin wait for all outstanding loads; it has no register
 // output, and the kernel waits for its own transfers (wait_transfers) before the barrier that publishes them.
+// The s_nop is the wait state a transfer needs behind a scalar write of m0 (the compiler adds it for the builtin, not
+// inside an asm block).  Naming the reserved m0 as clobbered is sound here because nothing else in the kernel uses it:
+// no builtin transfer, no indexed register move, no LDS access that is bounded by it.
 __device__ __forceinline__ void buffer_to_lds16(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
                  : "memory", "m0");
@@ -396,12 +399,12 @@ __device__ __forceinline__ void buffer_to_lds16(u32x4 rsrc, uint32_t voff, uint3
 template <int BYTES>
 __device__ __forceinline__ void buffer_to_lds(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
     if constexpr (BYTES == 2)
-        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_ushort %1, %2, %3 offen lds"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds"
                      :
                      : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
                      : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                      :
                      : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
                      : "memory", "m0");
