@@ -70,3 +70,13 @@ def test_rows_off_16_bytes_take_the_general_kernel():
                                            T, stride, dev(np.array([pos0], np.int32)).ptr, out.ptr, stride, None))
     got = out.download(np.float32, T * stride).reshape(T, stride)[:, :nq * hd].reshape(q.shape)
     assert np.abs(got - want64(q, gate, kc, vc, pos0)).max() <= ATOL
+
+
+@pytest.mark.parametrize("nq,nkv,hd,T,pos0", [
+    (32, 8, 128, 2, 0), (32, 8, 128, 8, 24), (32, 8, 128, 8, 25), (32, 8, 128, 12, 200), (8, 8, 128, 64, 0),
+    (5, 1, 128, 30, 2), (32, 8, 128, 260, 0), (16, 4, 256, 2, 0), (16, 4, 256, 8, 24), (16, 4, 256, 8, 56),
+    (16, 4, 256, 3, 110), (4, 4, 256, 64, 1)])
+def test_short_contexts(nq, nkv, hd, T, pos0):
+    """One to a few key tiles: the waves without a key are left out of the merge (edges of 32 keys, of a chunk, of the
+    tokens and heads of a block)."""
+    test_matches_64_bit_attention(nq, nkv, hd, T, pos0, 1.0)

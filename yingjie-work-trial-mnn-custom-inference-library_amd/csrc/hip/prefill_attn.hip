@@ -127,9 +127,15 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
 // (half the LDS bandwidth), and the online softmax's VALU work is about as long
 // as the MFMA work, so two waves per SIMD overlap the two.
 //
+// A short context's time is the chain around the keys.  q is read from memory once per block, in whole rows, and
+// handed out through LDS: read by every wave in operand order (32 columns x 64 bytes an instruction) it took 3 us.
+// Waves without a key neither write outputs nor are merged.
+//
 // Measured: 512 tokens after 3584, 32 / 8 heads of 128: 76 us (the kernel
 // before, one wave per query head of 16 tokens with no key split, 181 us);
-// 333 tokens after 512, 16 / 4 heads of 256: 42 us (prefill_attn_kernel 3603 us).
+// 16 tokens after 0: 7.5 us (9.1; 10.7 with q in operand order and all eight
+// waves merged); 333 tokens after 512, 16 / 4 heads of 256: 41 us
+// (prefill_attn_kernel 3603 us).
 constexpr int kFTile = 32;  // keys and columns of an MFMA tile
 
 template <int HD, int CT, int KS>
@@ -141,11 +147,17 @@ struct FlashTile {
     static constexpr int kLdo = HD + 4;   // floats per column of a wave's output
     static constexpr int kRowPieces = HD / 8;
     static constexpr int kPieces = kKeys * kRowPieces / kThreads;  // 16-byte pieces of K (or V) per thread and chunk
+    static constexpr int kTilePieces = kPieces / KS;               // ... and 32-key tile
+    static constexpr int kQuads = HD / 4;                          // float4 of an output row
+    static constexpr int kMergeCols = kThreads / kQuads;           // columns per pass of the merge
+    static constexpr int kPasses = kCols / kMergeCols;
     static constexpr size_t kKvBytes = static_cast<size_t>(kKeys) * (kLdk + kLdv) * 2;
     static constexpr size_t kOutBytes = static_cast<size_t>(kWaves) * kFTile * (kLdo + 2) * 4;
     static constexpr size_t kLds = kKvBytes > kOutBytes ? kKvBytes : kOutBytes;
-    static_assert(kPieces * kThreads == kKeys * kRowPieces, "K / V staging");
+    static_assert(kTilePieces * KS * kThreads == kKeys * kRowPieces, "K / V staging");
+    static_assert(kPasses * kThreads == kCols * kQuads, "merge");
     static_assert(kLds <= 160 * 1024, "LDS");
+    static_assert(static_cast<size_t>(kKeys) * kLdk * 2 + static_cast<size_t>(kCols) * kLdo * 4 <= kLds, "q fits behind K");
 };
 
 // v[l ^ 32] paired with v[l]: the larger
@@ -184,8 +196,9 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
     const int ct = wid % CT, ks = wid / CT;
     const int cl = lane & 31, g = lane >> 5;
     const int pos0 = __builtin_amdgcn_readfirstlane(*p.pos0);
+    const uint32_t inv_t = (65535u + T) / T;  // c / T = c inv_t >> 16 for c < 64, T <= 64
     const int t0 = tile * T, ntok = min(T, p.tokens - t0);
-    const int col = ct * kFTile + cl, ch = col / T, ctok = col - ch * T;
+    const int col = ct * kFTile + cl, ch = static_cast<int>(col * inv_t >> 16), ctok = col - ch * T;
     const bool live = ch < group && ctok < ntok;
     const int qpos = live ? pos0 + t0 + ctok : -1;           // this column's last key
     const int first = pos0 + t0, last = pos0 + t0 + ntok - 1;  // keys every / any column of the block sees
@@ -210,27 +223,45 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
         for (int u = 0; u < F::kPieces; ++u)
             *reinterpret_cast<u32x4*>(d + (pk + u * kKeyStep) * ld + 8 * pd) = r[u];
     };
-    load(p.k_cache, 0, kr);
-
-    // q fragments: lane supplies dims 16 s + 8 g .. + 7 of its column (columns without a token read 0)
-    half8 qhi[kSteps], qlo[kSteps];
-    float sscale;  // score scale in the exponent of 2
+    // rows of q, the gate and the output: thread i takes float4 i % kQuads of columns i / kQuads, + kMergeCols, ...
+    auto place = [&](int tid, int u, int stride) {  // float offset of the pass's column from token t0, or -1
+        const int c = tid / F::kQuads + u * F::kMergeCols;
+        const int hc = static_cast<int>(c * inv_t >> 16), tc = c - hc * T;
+        return hc < group && tc < ntok ? tc * stride + (kh * group + hc) * HD + 4 * (tid % F::kQuads) : -1;
+    };
+    // q to LDS (V's, before it)
+    u32x4 qr[F::kPasses];
     {
         const __amdgpu_buffer_rsrc_t rq =
             buf_rsrc(p.q + static_cast<size_t>(t0) * p.q_stride, static_cast<uint32_t>(ntok) * p.q_stride * 4u);
-        const uint32_t qoff = live ? static_cast<uint32_t>(ctok) * p.q_stride * 4u + ((kh * group + ch) * HD + 8 * g) * 4u
-                                   : kBufOOB;
+#pragma unroll
+        for (int u = 0; u < F::kPasses; ++u) {  // columns without a token read 0
+            const int at = place(threadIdx.x, u, p.q_stride);
+            qr[u] = __builtin_amdgcn_raw_buffer_load_b128(rq, at >= 0 ? static_cast<uint32_t>(at) * 4u : kBufOOB, 0, 0);
+        }
+    }
+    load(p.k_cache, 0, kr);
+    float* Ql = reinterpret_cast<float*>(Vl);  // [kCols][kLdo]
+#pragma unroll
+    for (int u = 0; u < F::kPasses; ++u)
+        *reinterpret_cast<u32x4*>(Ql + (threadIdx.x / F::kQuads + u * F::kMergeCols) * F::kLdo +
+                                  4 * (threadIdx.x % F::kQuads)) = qr[u];
+    store(Kl, F::kLdk, kr);
+    __syncthreads();
+    half8 qhi[kSteps], qlo[kSteps];  // lane supplies dims 16 s + 8 g .. + 7 of its column
+    float sscale;                    // score scale in the exponent of 2
+    {
         float x[kSteps][8], mx = 0.0f;
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            const auto a = __builtin_amdgcn_raw_buffer_load_b128(rq, qoff, 64 * s, 0);
-            const auto b = __builtin_amdgcn_raw_buffer_load_b128(rq, qoff, 64 * s + 16, 0);
+        for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                x[s][e] = __uint_as_float(a[e]);
-                x[s][4 + e] = __uint_as_float(b[e]);
+            for (int e = 0; e < 8; e += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(Ql + col * F::kLdo + 16 * s + 8 * g + e);
+                x[s][e] = v.x;
+                x[s][e + 1] = v.y;
+                x[s][e + 2] = v.z;
+                x[s][e + 3] = v.w;
             }
-        }
 #pragma unroll
         for (int s = 0; s < kSteps; ++s)
 #pragma unroll
@@ -249,12 +280,11 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
             split_h8(x[s], qhi[s], qlo[s]);
         }
     }
+    __syncthreads();  // every wave has its q: V may take its place
     float m = -1.0e30f, l = 0.0f;  // reference of the exponents, this lane's part of the sum
     floatx16 o[kDimTiles];
 #pragma unroll
     for (int j = 0; j < kDimTiles; ++j) o[j] = floatx16{};
-    store(Kl, F::kLdk, kr);
-    __syncthreads();
     for (int c0 = 0; c0 <= last; c0 += F::kKeys) {  // block-uniform
         load(p.v_cache, c0, vr);
         const int key0 = c0 + ks * kFTile;
@@ -302,7 +332,9 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
             }
         }
         store(Vl, F::kLdv, vr);
-        load(p.k_cache, c0 + F::kKeys, kr);
+        // block-uniform; 256 dims load on (past `last`: nothing is read): the branch costs them spilled registers
+        const bool more = HD > 128 || c0 + F::kKeys <= last;
+        if (more) load(p.k_cache, c0 + F::kKeys, kr);
         __syncthreads();  // V is staged; every wave has read K
         if (any) {
             // transposed reads: 16 lanes cover four keys x 16 dims, lane i gets dim i of the four
@@ -320,14 +352,26 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
                     o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, plo[h], o[j], 0, 0, 0);
                 }
         }
-        store(Kl, F::kLdk, kr);
+        if (more) store(Kl, F::kLdk, kr);
         __syncthreads();  // the next K is staged; every wave has read V
     }
-    // merge the KS key splits of each column tile: outputs, then (reference, sum) of every wave's columns
+    // merge the key splits of each column tile that have a key: outputs, then (reference, sum) of every wave's
+    // columns.  The gates are requested before the outputs go to LDS, so that no load waits behind a store.
+    const int splits = min(KS, last / kFTile + 1);
+    const __amdgpu_buffer_rsrc_t rg =
+        buf_rsrc(p.gate + static_cast<size_t>(t0) * p.q_stride, static_cast<uint32_t>(ntok) * p.q_stride * 4u);
+    int mt = threadIdx.x;
+    asm("" : "+v"(mt));  // (else the passes' places are kept from q's on, in registers that the loop needs)
+    u32x4 gate[F::kPasses];
+#pragma unroll
+    for (int u = 0; u < F::kPasses; ++u) {
+        const int at = place(mt, u, p.q_stride);
+        gate[u] = __builtin_amdgcn_raw_buffer_load_b128(rg, at >= 0 ? static_cast<uint32_t>(at) * 4u : kBufOOB, 0, 0);
+    }
     float* Ol = reinterpret_cast<float*>(flash_lds);  // [kWaves][32][kLdo]
     float* Ml = Ol + F::kWaves * kFTile * F::kLdo;    // [kWaves][32][2]
     l = xor_pair_sum<32>(l);
-    {
+    if (ks < splits) {
         float* oc = Ol + (wid * kFTile + cl) * F::kLdo + 4 * g;
 #pragma unroll
         for (int j = 0; j < kDimTiles; ++j)
@@ -335,39 +379,43 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
             for (int a = 0; a < 4; ++a)
                 *reinterpret_cast<float4*>(oc + 32 * j + 8 * a) =
                     make_float4(o[j][4 * a], o[j][4 * a + 1], o[j][4 * a + 2], o[j][4 * a + 3]);
-        if (g == 0) {
-            Ml[(wid * kFTile + cl) * 2] = m;
-            Ml[(wid * kFTile + cl) * 2 + 1] = l;
-        }
+        if (g == 0) *reinterpret_cast<float2*>(Ml + (wid * kFTile + cl) * 2) = make_float2(m, l);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < F::kCols * (HD / 4); i += F::kThreads) {
-        const int c = i / (HD / 4), d = 4 * (i % (HD / 4));
-        const int hc = c / T, tc = c - hc * T;
-        if (hc >= group || tc >= ntok) continue;
-        const int w0 = (c / kFTile) * kFTile + (c % kFTile);  // column c of wave (ct, ks): w0 + ks CT 32
-        float M = -INFINITY;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) M = fmaxf(M, Ml[(w0 + s * F::kCols) * 2]);
+    for (int u = 0; u < F::kPasses; ++u) {
+        const int at = place(mt, u, p.out_stride);
+        if (at < 0) continue;
+        const int c = mt / F::kQuads + u * F::kMergeCols;
+        const int w0 = (c / kFTile) * kFTile + (c % kFTile);  // column c of wave (ct, ks): w0 + ks CT 32
+        float ml[KS], ll[KS], M = -INFINITY;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            if (s < splits) {
+                const float2 v = *reinterpret_cast<const float2*>(Ml + (w0 + s * F::kCols) * 2);
+                ml[s] = v.x;
+                ll[s] = v.y;
+                M = fmaxf(M, v.x);
+            }
         float L = 0.0f;
         float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const int w = w0 + s * F::kCols;
-            const float f = exp2f(Ml[w * 2] - M);
-            const float4 v = *reinterpret_cast<const float4*>(Ol + w * F::kLdo + d);
-            L += f * Ml[w * 2 + 1];
-            r.x += f * v.x;
-            r.y += f * v.y;
-            r.z += f * v.z;
-            r.w += f * v.w;
-        }
+        for (int s = 0; s < KS; ++s)
+            if (s < splits) {
+                const float f = exp2f(ml[s] - M);
+                const float4 v = *reinterpret_cast<const float4*>(Ol + (w0 + s * F::kCols) * F::kLdo + 4 * (mt % F::kQuads));
+                L += f * ll[s];
+                r.x += f * v.x;
+                r.y += f * v.y;
+                r.z += f * v.z;
+                r.w += f * v.w;
+            }
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;  // custom_model.cpp:901-904
-        const size_t head = static_cast<size_t>(kh * group + hc) * HD + d;
-        const float4 gv = *reinterpret_cast<const float4*>(p.gate + static_cast<size_t>(t0 + tc) * p.q_stride + head);
-        *reinterpret_cast<float4*>(p.out + static_cast<size_t>(t0 + tc) * p.out_stride + head) =
-            make_float4((r.x * inv) * sigmoid_dev(gv.x), (r.y * inv) * sigmoid_dev(gv.y),
-                        (r.z * inv) * sigmoid_dev(gv.z), (r.w * inv) * sigmoid_dev(gv.w));
+        *reinterpret_cast<float4*>(p.out + static_cast<size_t>(t0) * p.out_stride + at) =
+            make_float4((r.x * inv) * sigmoid_dev(__uint_as_float(gate[u][0])),
+                        (r.y * inv) * sigmoid_dev(__uint_as_float(gate[u][1])),
+                        (r.z * inv) * sigmoid_dev(__uint_as_float(gate[u][2])),
+                        (r.w * inv) * sigmoid_dev(__uint_as_float(gate[u][3])));
     }
 }
 
@@ -391,11 +439,12 @@ static hipError_t launch_flash(const PrefillAttnLaunch& p, hipStream_t s) {
 
 hipError_t launch_prefill_attn(const PrefillAttnLaunch& p, hipStream_t s) {
     const int group = p.nq / p.nkv;
-    // the matrix-core kernel reads q, the gate and the output as 16-byte pieces
+    // the matrix-core kernel takes q, the gate, the output and the caches in 16-byte pieces
     const bool al16 = ((reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.gate) |
-                        reinterpret_cast<uintptr_t>(p.out) | reinterpret_cast<uintptr_t>(p.k_cache) |
-                        reinterpret_cast<uintptr_t>(p.v_cache)) & 15u) == 0 && p.q_stride % 4 == 0 && p.out_stride % 4 == 0;
-    if (al16 && (p.head_dim == 128 || p.head_dim == 256)) {
+                        reinterpret_cast<uintptr_t>(p.out)) & 15u) == 0 && p.q_stride % 4 == 0 && p.out_stride % 4 == 0 &&
+                      ((reinterpret_cast<uintptr_t>(p.k_cache) | reinterpret_cast<uintptr_t>(p.v_cache)) & 15u) == 0;
+    const bool in32 = p.q_stride < 1 << 24 && p.out_stride < 1 << 24;  // offsets within a block's (at most 64) rows
+    if (al16 && in32 && (p.head_dim == 128 || p.head_dim == 256)) {
         // two column tiles per block halve the K / V traffic per column; one tile with twice the key splits
         // where two would leave some of the 256 CUs without a block
         const bool wide = static_cast<long>((p.tokens + 64 / group - 1) / (64 / group)) * p.nkv >= 256;

@@ -260,13 +260,10 @@ __device__ __forceinline__ float block_sum_t(float v, float* red) {
 
 __device__ __forceinline__ float silu_dev(float x) { return x / (1.0f + expf(-x)); }
 
+// 1 / (1 + exp(-x)) for x >= 0, exp(x) / (1 + exp(x)) below, with the one exp they share
 __device__ __forceinline__ float sigmoid_dev(float x) {
-    if (x >= 0.0f) {
-        const float e = expf(-x);
-        return 1.0f / (1.0f + e);
-    }
-    const float e = expf(x);
-    return e / (1.0f + e);
+    const float e = expf(-fabsf(x));
+    return (x >= 0.0f ? 1.0f : e) / (1.0f + e);
 }
 
 __device__ __forceinline__ float softplus_dev(float x) {
