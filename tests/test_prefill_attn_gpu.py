@@ -6,6 +6,8 @@ of its tiles: 32- and 64-column blocks (tokens x query heads of a kv head), the
 Bound: q and the probabilities carry about 22 bits (fp16 hi + lo), so a score of
 |q| |k| / sqrt(hd) <= 16 is off by at most 16 x 2^-22 and a probability by 4e-6
 of itself; the output, a convex combination of |v| <= 6, by 3e-5."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -80,3 +82,20 @@ def test_short_contexts(nq, nkv, hd, T, pos0):
     """One to a few key tiles: the waves without a key are left out of the merge (edges of 32 keys, of a chunk, of the
     tokens and heads of a block)."""
     test_matches_64_bit_attention(nq, nkv, hd, T, pos0, 1.0)
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(8, 2, 128), (8, 2, 256)])
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_caches_off_16_bytes(nq, nkv, hd, shift):
+    """Caches that start 2, 4 or 8 bytes into an allocation."""
+    T, pos0 = 19, 41
+    rng = np.random.default_rng(shift)
+    kc, vc = (rng.normal(0, 1, (pos0 + T, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.normal(0, 1, (T, nq, hd)).astype(np.float32) for _ in range(2))
+    k, v = (dev(np.concatenate([np.zeros(shift, np.float16), a.reshape(-1)])) for a in (kc, vc))
+    at = lambda b: ctypes.c_void_p(b.ptr.value + 2 * shift)  # noqa: E731
+    out = xb.DeviceBuffer(q.nbytes)
+    xb.ck(xb.hip().xqhip_prefill_attention(dev(q).ptr, dev(gate).ptr, at(k), at(v), nq, nkv, hd, T, nq * hd,
+                                           dev(np.array([pos0], np.int32)).ptr, out.ptr, nq * hd, None))
+    got = out.download(np.float32, q.size).reshape(q.shape)
+    assert np.abs(got - want64(q, gate, kc, vc, pos0)).max() <= ATOL

@@ -439,10 +439,10 @@ static hipError_t launch_flash(const PrefillAttnLaunch& p, hipStream_t s) {
 
 hipError_t launch_prefill_attn(const PrefillAttnLaunch& p, hipStream_t s) {
     const int group = p.nq / p.nkv;
-    // the matrix-core kernel takes q, the gate, the output and the caches in 16-byte pieces
+    // the matrix-core kernel takes q, the gate and the output in 16-byte pieces, the caches in whole words
     const bool al16 = ((reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.gate) |
                         reinterpret_cast<uintptr_t>(p.out)) & 15u) == 0 && p.q_stride % 4 == 0 && p.out_stride % 4 == 0 &&
-                      ((reinterpret_cast<uintptr_t>(p.k_cache) | reinterpret_cast<uintptr_t>(p.v_cache)) & 15u) == 0;
+                      ((reinterpret_cast<uintptr_t>(p.k_cache) | reinterpret_cast<uintptr_t>(p.v_cache)) & 3u) == 0;
     const bool in32 = p.q_stride < 1 << 24 && p.out_stride < 1 << 24;  // offsets within a block's (at most 64) rows
     if (al16 && in32 && (p.head_dim == 128 || p.head_dim == 256)) {
         // two column tiles per block halve the K / V traffic per column; one tile with twice the key splits
