@@ -99,3 +99,45 @@ def test_caches_off_16_bytes(nq, nkv, hd, shift):
                                            dev(np.array([pos0], np.int32)).ptr, out.ptr, nq * hd, None))
     got = out.download(np.float32, q.size).reshape(q.shape)
     assert np.abs(got - want64(q, gate, kc, vc, pos0)).max() <= ATOL
+
+
+SHAPES = [(16, 4, 256, 40, 3), (4, 4, 256, 9, 130), (32, 8, 128, 512, 0), (3, 1, 128, 33, 60), (16, 2, 128, 21, 300)]
+
+
+def attend(q, gate, kc, vc, pos0):
+    T, nq, hd = q.shape
+    out = dev(np.full((T, nq * hd), 7.0, np.float32))
+    # (the buffers live until the download: the launch does not wait)
+    args = [dev(a) for a in (q, gate, kc, vc, np.array([pos0], np.int32))]
+    xb.ck(xb.hip().xqhip_prefill_attention(args[0].ptr, args[1].ptr, args[2].ptr, args[3].ptr, nq, kc.shape[1], hd, T,
+                                           nq * hd, args[4].ptr, out.ptr, nq * hd, None))
+    return out.download(np.float32, T * nq * hd).reshape(q.shape)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("nq,nkv,hd,T,pos0", SHAPES)
+def test_a_value_that_is_not_finite_reaches_its_own_and_later_tokens_only(nq, nkv, hd, T, pos0, value):
+    """A value beyond fp16's range is an infinity in the cache: tokens before it are as if it were not there, its own
+    and later ones get it in that dim."""
+    rng = np.random.default_rng(T + pos0)
+    kc, vc = (rng.normal(0, 1, (pos0 + T, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.normal(0, 1, (T, nq, hd)).astype(np.float32) for _ in range(2))
+    want = want64(q, gate, kc, vc, pos0)
+    t, kh, d = T - 3, nkv - 1, hd - 5
+    vc[pos0 + t, kh, d] = value
+    got = attend(q, gate, kc, vc, pos0)
+    heads, group = slice(kh * nq // nkv, None), nq // nkv
+    assert group == got[:, heads].shape[1]
+    np.testing.assert_array_equal(got[t:, heads, d], np.full((T - t, group), value, np.float32))
+    want[t:, heads, d] = got[t:, heads, d] = 0.0
+    assert np.abs(got - want).max() <= ATOL
+
+
+@pytest.mark.parametrize("nq,nkv,hd,T,pos0", SHAPES)
+def test_scores_near_the_lowest_value(nq, nkv, hd, T, pos0):
+    """All scores -1e30 sqrt(hd), as a mask of large negative queries gives: the mean of the values."""
+    rng = np.random.default_rng(T + pos0)
+    vc = rng.normal(0, 1, (pos0 + T, nkv, hd)).astype(np.float16)
+    q, gate = np.full((T, nq, hd), -1e30, np.float32), np.zeros((T, nq, hd), np.float32)
+    got = attend(q, gate, np.ones_like(vc), vc, pos0)
+    assert np.abs(got - want64(q, gate, np.ones_like(vc), vc, pos0)).max() <= ATOL

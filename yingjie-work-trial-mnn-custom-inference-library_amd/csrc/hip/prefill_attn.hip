@@ -15,7 +15,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
-// Causal GQA for a prompt chunk: block (t, kh) takes query token t (position
+// Causal GQA for a prompt chunk: a block takes query token t (position
 // pos0 + t) and the `group` query heads of kv head kh over keys 0..pos0+t in
 // 64-token chunks with a running max / sum (rescaled by exp(m_old - m_new)),
 // then normalises by multiplying with 1/l and applies the sigmoid gate
@@ -24,9 +24,15 @@ typedef short short4_t __attribute__((ext_vector_type(4)));
 constexpr int kPAttnChunk = 64;
 constexpr int kPAttnMaxGroup = 8;
 
-__global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) {
-    extern __shared__ float smem[];
-    const int t = blockIdx.x, kh = blockIdx.y;
+// floats of LDS of attend_token
+constexpr size_t attend_token_lds(int group, int hd) {
+    return 2 * static_cast<size_t>(group) * hd + static_cast<size_t>(group) * (kPAttnChunk + 3);
+}
+
+// THREADS: of the block (a constant: blockDim would add the implicit arguments to every launch's)
+template <int THREADS>
+__device__ __forceinline__ void attend_token(const PrefillAttnLaunch& p, int t, int kh, float* smem) {
+    static_assert(THREADS >= 4 * kPAttnChunk, "four threads per key");
     const int hd = p.head_dim, group = p.nq / p.nkv;
     const int ctx = *p.pos0 + t + 1;
     float* qs = smem;                        // [group][hd]
@@ -35,7 +41,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
     float* ml = osum + group * hd;           // [group][2] running max, sum
     float* fac = ml + 2 * group;             // [group] rescale of this chunk
     const float* qrow = p.q + static_cast<size_t>(t) * p.q_stride + static_cast<size_t>(kh) * group * hd;
-    for (int i = threadIdx.x; i < group * hd; i += blockDim.x) {
+    for (int i = threadIdx.x; i < group * hd; i += THREADS) {
         qs[i] = qrow[i];
         osum[i] = 0.0f;
     }
@@ -63,7 +69,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
         }
         __syncthreads();
         // online softmax update per head (one wave per head)
-        for (int g = wid; g < group; g += blockDim.x / kWave) {
+        for (int g = wid; g < group; g += THREADS / kWave) {
             const float sv = lane < n ? sc[g * kPAttnChunk + lane] : -INFINITY;
             const float mc = wave_max(sv);
             const float m_old = ml[2 * g];
@@ -79,7 +85,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
             }
         }
         __syncthreads();
-        for (int i = threadIdx.x; i < group * hd; i += blockDim.x) {
+        for (int i = threadIdx.x; i < group * hd; i += THREADS) {
             const int g = i / hd, d = i % hd;
             float o = osum[i] * fac[g];
             for (int j = 0; j < n; ++j)
@@ -89,7 +95,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
         }
         __syncthreads();
     }
-    for (int i = threadIdx.x; i < group * hd; i += blockDim.x) {
+    for (int i = threadIdx.x; i < group * hd; i += THREADS) {
         const int g = i / hd;
         const float l = ml[2 * g + 1];
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
@@ -99,6 +105,10 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
     }
 }
 
+__global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) {
+    extern __shared__ float smem[];
+    attend_token<256>(p, blockIdx.x, blockIdx.y, smem);
+}
 
 // Matrix-core form.  A block takes 32 CT columns of one kv head, a column
 // being one (token, query head) pair: column c is head c / T of the kv head's
@@ -119,7 +129,13 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
 // Precision: q (scaled per column by a power of two to [2^12, 2^13), exact)
 // and p (relative to a reference within 2^6 of the column's running max, times
 // 2^6) are split into fp16 hi + lo, about 22 bits together; k and v are fp16
-// in the cache; fp32 accumulation.
+// in the cache; fp32 accumulation.  (prefill_attn_kernel holds q and p in fp32; both are within 2^-22 of their
+// value here, and the output, against 64 bits over normal data, is nearer: 2.8e-7 of its norm against 5.1e-7 at 333
+// tokens after 512, 16 / 4 heads of 256.)
+//
+// A masked key has weight 0, but 0 times an infinity is not 0, and neither hi + lo nor the finite start of the running
+// max can carry infinities or scores below -1e30.  Where that happens the output is not finite or its weights sum to
+// 0: a block that finds such an output (one flag, read once at its end) computes its tokens again by attend_token.
 //
 // What bounds it: MFMA work is 8 pairs x hd x 2 passes of flops (q hi / lo, p hi
 // / lo), 65 GFLOP at 512 tokens over 4096 keys and 32 heads; the 32-column
@@ -156,8 +172,9 @@ struct FlashTile {
     static constexpr size_t kLds = kKvBytes > kOutBytes ? kKvBytes : kOutBytes;
     static_assert(kTilePieces * KS * kThreads == kKeys * kRowPieces, "K / V staging");
     static_assert(kPasses * kThreads == kCols * kQuads, "merge");
-    static_assert(kLds <= 160 * 1024, "LDS");
+    static_assert(kLds + 64 <= 160 * 1024, "LDS");
     static_assert(static_cast<size_t>(kKeys) * kLdk * 2 + static_cast<size_t>(kCols) * kLdo * 4 <= kLds, "q fits behind K");
+    static_assert(kLds >= attend_token_lds(kPAttnMaxGroup, HD) * 4, "the general form runs in it");
 };
 
 // v[l ^ 32] paired with v[l]: the larger
@@ -186,6 +203,7 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
     constexpr float kRaise = 6.0f;  // p is held times 2^kRaise
     constexpr float kSlack = 6.0f;  // the max may outgrow the reference by 2^kSlack before it is moved
     extern __shared__ uint4 flash_lds[];
+    __shared__ int redo;  // some output of the block is not finite
     _Float16* Kl = reinterpret_cast<_Float16*>(flash_lds);  // [kKeys][kLdk]
     _Float16* Vl = Kl + F::kKeys * F::kLdk;                 // [kKeys][kLdv]
     // the kv heads of a token tile are neighbours in launch order, so a head's blocks share an XCD's L2 (8
@@ -247,6 +265,7 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
         *reinterpret_cast<u32x4*>(Ql + (threadIdx.x / F::kQuads + u * F::kMergeCols) * F::kLdo +
                                   4 * (threadIdx.x % F::kQuads)) = qr[u];
     store(Kl, F::kLdk, kr);
+    if (threadIdx.x == 0) redo = 0;
     __syncthreads();
     half8 qhi[kSteps], qlo[kSteps];  // lane supplies dims 16 s + 8 g .. + 7 of its column
     float sscale;                    // score scale in the exponent of 2
@@ -382,6 +401,7 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
         if (g == 0) *reinterpret_cast<float2*>(Ml + (wid * kFTile + cl) * 2) = make_float2(m, l);
     }
     __syncthreads();
+    bool bad = false;
 #pragma unroll
     for (int u = 0; u < F::kPasses; ++u) {
         const int at = place(mt, u, p.out_stride);
@@ -411,17 +431,27 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
                 r.w += f * v.w;
             }
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;  // custom_model.cpp:901-904
+        bad |= !(L > 0.0f && fabsf(r.x) + fabsf(r.y) + fabsf(r.z) + fabsf(r.w) < INFINITY);
         *reinterpret_cast<float4*>(p.out + static_cast<size_t>(t0) * p.out_stride + at) =
             make_float4((r.x * inv) * sigmoid_dev(__uint_as_float(gate[u][0])),
                         (r.y * inv) * sigmoid_dev(__uint_as_float(gate[u][1])),
                         (r.z * inv) * sigmoid_dev(__uint_as_float(gate[u][2])),
                         (r.w * inv) * sigmoid_dev(__uint_as_float(gate[u][3])));
     }
+    if (bad) redo = 1;
+    // a barrier for the flag alone: __syncthreads() would wait for the output stores too (1 us)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+    if (__builtin_expect(!redo, 1)) return;  // block-uniform
+    __syncthreads();  // those stores, and every wave's reads of the LDS used again
+    for (int t = t0; t < t0 + ntok; ++t) {
+        attend_token<F::kThreads>(p, t, kh, reinterpret_cast<float*>(flash_lds));
+        __syncthreads();
+    }
 }
 
 bool prefill_attn_supported(int nq, int nkv, int head_dim) {
     return nkv > 0 && nq % nkv == 0 && nq / nkv <= kPAttnMaxGroup && head_dim > 0 &&
-           sizeof(float) * (2 * (nq / nkv) * head_dim + (nq / nkv) * (kPAttnChunk + 3)) <= 64 * 1024;
+           sizeof(float) * attend_token_lds(nq / nkv, head_dim) <= 64 * 1024;
 }
 
 template <int HD, int CT, int KS>
@@ -451,7 +481,7 @@ hipError_t launch_prefill_attn(const PrefillAttnLaunch& p, hipStream_t s) {
         if (p.head_dim == 128) return wide ? launch_flash<128, 2, 4>(p, s) : launch_flash<128, 1, 8>(p, s);
         return wide ? launch_flash<256, 2, 2>(p, s) : launch_flash<256, 1, 4>(p, s);
     }
-    const size_t lds = sizeof(float) * (2 * static_cast<size_t>(group) * p.head_dim + group * (kPAttnChunk + 3));
+    const size_t lds = sizeof(float) * attend_token_lds(group, p.head_dim);
     hipLaunchKernelGGL(prefill_attn_kernel, dim3(p.tokens, p.nkv), dim3(256), lds, s, p);
     return hipGetLastError();
 }
