@@ -69,3 +69,28 @@ def test_matches_64_bit_product(rows, cols, m, epi, form):
         tol = tol + 2.0**-23 * np.abs(y)
     err = np.abs(got[:, :out] - y)
     assert (err <= tol).all(), (err / tol).max()
+
+
+@pytest.mark.parametrize("rows,cols,m", [(256, 512, 3), (128, 4096, 2), (24600, 128, 500), (20002, 128, 257)])
+def test_columns_beside_an_outlier(rows, cols, m):
+    """One weight a row beside a token's outlier of 2^14 times the other values (under the zero point): scaled with the
+    outlier to 2^12 .. 2^13, x is off by 2^-22 of itself and 2^-25 (half the smallest fp16) = 2^-37 of the outlier, the
+    same in even and odd columns; the sum of hi and lo, the scale and the result round to fp32."""
+    rng = np.random.default_rng(cols)
+    r = np.arange(rows)
+    q = np.full((rows, cols), 8, np.uint8)
+    at = 1 + r % (cols - 1)
+    q[r, at] = (8 + rng.integers(1, 16, rows)) % 16
+    scales = np.abs(rng.normal(0, 0.02, rows * cols // 64)).astype(np.float16).astype(np.float32)
+    w = xb.DeviceW4(q[:, 0::2] | q[:, 1::2] << 4, scales, np.full_like(scales, 8.0), rows, cols)
+    x = rng.normal(0, 1, (m, cols)).astype(np.float32)
+    x[:, 0] = 2.0**14
+    yd, xd = xb.DeviceBuffer(4 * m * rows), dev(x)
+    ws = xb.DeviceBuffer(xb.hip().xqhip_gemm_workspace_bytes(m, cols, rows))
+    xb.ck(xb.hip().xqhip_gemm_w4a16(w.ref, xd.ptr, m, cols, None, 0, yd.ptr, rows, xb.EPI_STORE, ws.ptr, ws.nbytes, None))
+    got = yd.download(np.float32, m * rows).reshape(m, rows)
+    weight = (q[r, at].astype(np.float64) - 8) * scales.reshape(rows, -1)[r, at // 64]
+    xa = x[:, at].astype(np.float64)
+    tol = np.abs(weight) * (np.abs(xa) * (2.0**-22 + 3 * 2.0**-24) + 2.0**(14 - 37))
+    err = np.abs(got - weight * xa)
+    assert (err <= tol).all(), (err / tol).max()

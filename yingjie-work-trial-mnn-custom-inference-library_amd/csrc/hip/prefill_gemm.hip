@@ -134,12 +134,10 @@ __global__ void __launch_bounds__(256) prep_x_kernel(const float* __restrict__ x
         float sum = 0.0f;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {  // positions 2p, 2p + 1 <- columns p, p + 4
-            const float down16 = p & 1 ? 0.0625f : 1.0f;  // codes 1, 3, 5, 7 are unpacked times 16
-            const float va = v[p] * down16, vb = v[p + 4] * down16;
-            const _Float16 ha = static_cast<_Float16>(va), hb = static_cast<_Float16>(vb);
+            const _Float16 ha = static_cast<_Float16>(v[p]), hb = static_cast<_Float16>(v[p + 4]);
             ph[p] = pack_h2(ha, hb);
-            pl[p] = pack_h2(static_cast<_Float16>(va - static_cast<float>(ha)),
-                            static_cast<_Float16>(vb - static_cast<float>(hb)));
+            pl[p] = pack_h2(static_cast<_Float16>(v[p] - static_cast<float>(ha)),
+                            static_cast<_Float16>(v[p + 4] - static_cast<float>(hb)));
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) sum += v[e];
@@ -263,12 +261,10 @@ __global__ void __launch_bounds__(256) prep_x_vec_kernel(const float* __restrict
         for (int e = 0; e < 8; ++e) v[k][e] *= down;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {  // positions 2q, 2q + 1 <- columns q, q + 4
-            const float down16 = q & 1 ? 0.0625f : 1.0f;  // codes 1, 3, 5, 7 are unpacked times 16
-            const float va = v[k][q] * down16, vb = v[k][q + 4] * down16;
-            const _Float16 ha = static_cast<_Float16>(va), hb = static_cast<_Float16>(vb);
+            const _Float16 ha = static_cast<_Float16>(v[k][q]), hb = static_cast<_Float16>(v[k][q + 4]);
             ph[q] = pack_h2(ha, hb);
-            pl[q] = pack_h2(static_cast<_Float16>(va - static_cast<float>(ha)),
-                            static_cast<_Float16>(vb - static_cast<float>(hb)));
+            pl[q] = pack_h2(static_cast<_Float16>(v[k][q] - static_cast<float>(ha)),
+                            static_cast<_Float16>(v[k][q + 4] - static_cast<float>(hb)));
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) sum += v[k][e];
@@ -309,8 +305,8 @@ static bool prep_vec_ok(const GemmLaunch& p) {
 // w = (q - z) s, or 8 s + z for w = q s + z.  Hence
 //     y[t][r] = sum_g s[r][g] A[r][t][g] + sum_g c0[r][g] xs[t][g],
 //     A[r][t][g] = sum_{k in g} sn[r][k] x[t][k],  xs[t][g] = sum_{k in g} x[t][k].
-// sn is exact in fp16, so A takes two v_mfma_f32_32x32x16_f16 passes (sn x_hi +
-// sn x_lo) into a per-group accumulator, which is scaled by s into the fp32
+// 16 sn is exact in fp16, so 16 A takes two v_mfma_f32_32x32x16_f16 passes (x_hi and
+// x_lo) into a per-group accumulator, which is scaled by s into the fp32
 // result.  The c0 term is a K = G contraction done after the group loop in
 // three fp16 hi/lo passes (c0 scaled by 64 and xs by 1/64, both exact, to stay
 // in fp16 range), skipped where every zero is 8.
@@ -370,16 +366,18 @@ struct GemmTile {
     static_assert(kXU * kThreads == kBT * 16 && kAU * kThreads == kBR * 4 && kSU * kThreads == kBR * 4, "staging");
 };
 
-// 8 stored codes (q ^ 8; column n of the word in bits 4n..4n+3) -> fp16, in the
-// column order [0 4 1 5 2 6 3 7]: q - 8 for the even columns, 16 (q - 8) for the
-// odd ones (whose x is prepared divided by 16).  (w & 0x000F000F) ^ 0x64086408 is
-// fp16 1024 + q for codes 0 and 4, (w & 0x00F000F0) ^ 0x64806480 is 1024 + 16 q
-// for codes 1 and 5, and w >> 8 gives the other four.
+// 8 stored codes (q ^ 8; column n of the word in bits 4n..4n+3) -> fp16 16 (q - 8),
+// in the column order [0 4 1 5 2 6 3 7].  (w & 0x000F000F) ^ 0x74087408 is fp16
+// 16384 + 16 q for codes 0 and 4 (one step of fp16 there is 16), (w & 0x00F000F0) ^
+// 0x64806480 is 1024 + 16 q for codes 1 and 5, and w >> 8 gives the other four; both
+// differences are exact.  The 16 leaves the sums once, at the end: x is the same
+// fp16 pair in every column (held divided by 16 in the odd ones, for codes of q - 8
+// and 16 (q - 8), its lo half met fp16's subnormals 16 times earlier beside an outlier).
 template <int P>  // codes 2 P, 2 P + 1 of that order
 __device__ __forceinline__ uint32_t unpack_pair(uint32_t w) {
     const uint32_t v = P & 2 ? w >> 8 : w;
-    const _Float16 bias = static_cast<_Float16>(P & 1 ? 1152.0f : 1032.0f);
-    const uint32_t m = P & 1 ? (v & 0x00F000F0u) ^ 0x64806480u : (v & 0x000F000Fu) ^ 0x64086408u;
+    const _Float16 bias = static_cast<_Float16>(P & 1 ? 1152.0f : 16512.0f);
+    const uint32_t m = P & 1 ? (v & 0x00F000F0u) ^ 0x64806480u : (v & 0x000F000Fu) ^ 0x74087408u;
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, m) - half2_t{bias, bias});
 }
 
@@ -654,6 +652,10 @@ gemm_w4_mfma_kernel(GemmArgs a) {
     for (int q = 0; q < 4 * NP; ++q)
         if (scale_slot(q >> 2, q & 3) >= NM) scale_in(q >> 2, q & 3, 1);
     wait_transfers<0>();  // the last phase's requests, which nothing reads
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] *= 0.0625f;  // the codes' 16
 
     // c0 term: K = G, lane half h takes groups gb + 8 h + 0..7 of its token / row.  All loads of a step are
     // issued before any use; groups past g1 read out of range (zero), so c0 and xs are 0.
