@@ -38,8 +38,9 @@ def matrix(rng, rows, cols, form):
 @pytest.mark.parametrize("rows,cols,m,epi", [
     (128, 512, 1, "store"), (129, 1024, 32, "add"), (34, 4160, 33, "silu"), (1000, 640, 31, "store"),  # small tile
     (258, 2048, 7, "silu"), (96, 12288, 40, "add"),                                                    # ... split
-    (20001, 576, 130, "add"), (20000, 64, 129, "silu"), (24600, 320, 500, "store"),                     # middle tile
-    (20002, 192, 257, "store"), (19970, 448, 300, "add"), (20000, 256, 384, "silu")])                   # large tile
+    (20001, 576, 130, "add"), (20000, 64, 129, "silu"),                                                 # middle tile
+    (4098, 3648, 247, "silu"), (1502, 5952, 450, "add"),                                                # ... split
+    (24600, 320, 500, "store"), (20002, 192, 257, "store"), (19970, 448, 300, "add"), (20000, 256, 384, "silu")])  # large
 def test_matches_64_bit_product(rows, cols, m, epi, form):
     rng = np.random.default_rng(rows + cols + m)
     packed, scales, zeros, affine, W = matrix(rng, rows, cols, form)

@@ -428,6 +428,7 @@ template <int WGR, int WGT, int TI, int TJ, int XS, int META>
 __global__ void __launch_bounds__(kWave * WGR * WGT) __attribute__((amdgpu_waves_per_eu(TI * TJ <= 2 ? 4 : 2)))
 gemm_w4_mfma_kernel(GemmArgs a) {
     constexpr uint32_t kMetaBytes = kMetaGroupBytes<META>;
+    constexpr bool kSplits = WGR * WGT == 4;  // the 8-wave tile is never split over K (gemm_plan)
     using T = GemmTile<WGR, WGT, TI, TJ, XS>;
     constexpr int BR = T::kBR, BT = T::kBT, XU = T::kXU, AU = T::kAU, SU = T::kSU, NT = T::kThreads;
     extern __shared__ u32x4 gemm_lds[];
@@ -720,9 +721,9 @@ gemm_w4_mfma_kernel(GemmArgs a) {
     // epilogue: lane holds row lr of tile i and the tokens 8 (v >> 2) + 4 lh + (v & 3) of tile j
     auto finish = [&](auto whole) {  // whole: every row and token of the block exists
         constexpr bool kWhole = decltype(whole)::value;
-        const bool pair = a.epi == 2 && !a.part, add = a.epi == 1 && !a.part;
-        const size_t ld = a.part ? static_cast<size_t>(a.rows) : static_cast<size_t>(a.ldy);
-        float* out = a.part ? a.part + static_cast<size_t>(split) * a.m * a.rows : a.y;
+        const bool part = kSplits && a.part, pair = a.epi == 2 && !part, add = a.epi == 1 && !part;
+        const size_t ld = part ? static_cast<size_t>(a.rows) : static_cast<size_t>(a.ldy);
+        float* out = part ? a.part + static_cast<size_t>(split) * a.m * a.rows : a.y;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
             const int tb = t0 + 32 * (wj + j) + 4 * lh;
@@ -852,55 +853,46 @@ struct GemmPlan {
     int bt, splits, gps;  // tokens per block, K splits, column groups per split (a multiple of 4)
 };
 
-// Tile and K splits of a launch, from a sweep of rows 1024..24576, cols 2048..12288 and 4..512 tokens (both sides
-// in us, prep and reduce included):
-//   128 rows x 32 tokens (4 waves, 3 blocks per CU) while that gives at most 600 blocks: more blocks to hide each
-//     other's latency, no padding of short prompts.  12352x4096, 128 tokens 40 against 44 with 256 x 64;
-//     24576x4096, 128 tokens (768 blocks) 66 against 62.
-//   256 x 64 (4 waves, two blocks per CU, which do not wait at each other's barriers): 24576x4096, 512 tokens 186
-//     against 208 with 256 x 128.
-//   256 x 128 (8 waves, one block per CU) where 256 x 64 gives more than 256 but at most 512 blocks, a partly filled
-//     second block per CU: 12352x4096, 512 tokens 100 against 109; 24576x4096, 256 tokens 98 against 105.
-// Launches short of a block per CU split the column groups over blockIdx.z, and a second kernel adds the splits'
-// partial products in a fixed order (deterministic): 4096x4096, 8 tokens 16 us with 4 splits, 26 with one;
-// 4096x12288, 512 tokens 122 with 2, 167 with one.
+// us that a block spends on a group of 64 columns where `blocks` share the CUs: a part for each block of the fullest
+// CU and a part for the load of the whole chip (memory, power).  Fitted to 2000 launches: 512 to 24600 rows, 1024 to
+// 12288 columns, 2 to 512 tokens, every tile and split.  3 small or 2 middle blocks are resident on a CU at once.
+static double group_us(GemmTileKind tile, long blocks) {
+    const double per_cu = blocks / 256.0, n = static_cast<double>((blocks + 255) / 256);
+    if (tile == kTileMid) return 0.22 + 0.48 * n + 0.35 * per_cu;
+    if (tile == kTileLarge) return 0.05 + 1.02 * n + 0.43 * per_cu;
+    return n == 1 ? 0.30 + 0.11 * per_cu : n == 2 ? 0.37 + 0.16 * per_cu : n == 3 ? 0.43 + 0.23 * per_cu : 0.16 * n + 0.18 * per_cu;
+}
+
+// Tile and K splits of a launch: the least time by group_us, a split launch with its second kernel and the partial
+// products' traffic added.  That kernel adds the splits in a fixed order: deterministic.
+//   128 rows x 32 tokens (4 waves): the most blocks, no padding of short prompts.
+//   256 x 64 (4 waves): half the LDS reads per product.
+//   256 x 128 (8 waves, one block per CU): half the x again, where one round of blocks covers the launch.  Never
+//     split: with fewer blocks than CUs to split for, the middle tile has twice as many.
+// Measured, us with prep and reduce (small, middle, large tile; splits in brackets), the choice first:
+//   4096x4096, 8 tokens: small 15.4 (8), 24.5 (1).            24576x4096, 64: small 41.5 (1), 46.1 (2), middle 44.0 (2)
+//   24576x4096, 300: middle 118.6, small 160, large 182.       12352x4096, 512: large 99.5, middle 109, small 142
+//   24576x4096, 512: middle 181, large 195, small 246.         4096x12288, 512: middle 114 (2), 152 (1), small 136
+//   10240x10240, 128: middle 68 (3), 122 (1), small 88.
+// Over 240 sizes the choice is 1 % behind the fastest tile and split on average, 8 % at most.
 static GemmPlan gemm_plan(int rows, int m, int cols) {
     const int G = cols / 64;
     auto blocks = [&](int br, int bt) { return static_cast<long>((m + bt - 1) / bt) * ((rows + br - 1) / br); };
-    GemmPlan p{};
-    p.splits = 1;
-    long nb = blocks(128, 32);
-    if (nb <= 600) {
-        p.tile = kTileSmall;
-        p.bt = 32;
-        // Split while a group's time (us, for the blocks sharing a CU, as measured) times the groups left to a
-        // block outweighs the second kernel and the partial products' traffic.  2048x8192, 300 tokens (160 blocks):
-        // 46 us unsplit, 33 with 3.
-        auto per_group = [](double per_cu) {
-            return per_cu <= 1.0 ? 0.32 : per_cu <= 2.0 ? 0.12 + 0.2 * per_cu : per_cu <= 3.0 ? 0.28 * per_cu - 0.04 : 0.27 * per_cu;
-        };
-        double best = 1.0e30;
-        for (int s = 1; s <= std::min(kGemmMaxSplits, std::max(1, G / 8)); ++s) {
-            const double t = ((G + s - 1) / s + 3) / 4 * 4 * per_group(nb * s / 256.0) +
-                             (s > 1 ? 4.5 + 2.0e-6 * s * m * rows : 0.0);
-            if (t < best) {
-                best = t;
-                p.splits = s;
+    struct Option { GemmTileKind tile; int br, bt, splits; };
+    GemmPlan best{};
+    double least = 1.0e30;
+    for (const Option& o : {Option{kTileSmall, 128, 32, kGemmMaxSplits}, Option{kTileMid, 256, 64, 4}, Option{kTileLarge, 256, 128, 1}})
+        for (int s = 1; s <= std::min(o.splits, std::max(1, G / 8)); ++s) {  // at least two quads of groups per split
+            if (s > 1 && static_cast<size_t>(s) * m * rows > kGemmPartMax) break;  // the workspace's bound
+            const int gps = ((G + s - 1) / s + 3) / 4 * 4, splits = (G + gps - 1) / gps;
+            const double t = (gps + 5) * group_us(o.tile, blocks(o.br, o.bt) * splits) +  // 5: a block's start and end
+                             (splits > 1 ? 2.5 + 2.5e-6 * splits * m * rows : 0.0);
+            if (t < least) {
+                least = t;
+                best = GemmPlan{o.tile, o.bt, splits, gps};
             }
         }
-    } else {
-        nb = blocks(256, 64);
-        p.tile = nb > 256 && nb <= 512 ? kTileLarge : kTileMid;
-        p.bt = p.tile == kTileLarge ? 128 : 64;
-        if (p.tile == kTileLarge) nb = blocks(256, 128);
-        p.splits = static_cast<int>(256 / nb);
-    }
-    // at least two quads of groups per split, and the partial products within the workspace's bound
-    p.splits = std::max(1, std::min({p.splits, kGemmMaxSplits, G / 8}));
-    while (p.splits > 1 && static_cast<size_t>(p.splits) * m * rows > kGemmPartMax) --p.splits;
-    p.gps = ((G + p.splits - 1) / p.splits + 3) / 4 * 4;
-    p.splits = (G + p.gps - 1) / p.gps;
-    return p;
+    return best;
 }
 
 hipError_t launch_gemm(const GemmLaunch& p, hipStream_t s) {
