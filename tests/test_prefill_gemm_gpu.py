@@ -95,3 +95,36 @@ def test_columns_beside_an_outlier(rows, cols, m):
     tol = np.abs(weight) * (np.abs(xa) * (2.0**-22 + 3 * 2.0**-24) + 2.0**(14 - 37))
     err = np.abs(got - weight * xa)
     assert (err <= tol).all(), (err / tol).max()
+
+
+@pytest.mark.parametrize("cols,pro", [(640, "none"), (2048, "none"), (640, "rms"), (4096, "gated")])
+def test_rows_of_tiny_values(cols, pro):
+    """Rows whose largest magnitude is far below 2^-113, subnormal or 0: the row's power of two stays finite (fp16 then
+    holds 2^-152, below fp32's smallest), the result has the precision of any other row down to fp32's subnormals."""
+    rows, m = 96, 6
+    rng = np.random.default_rng(cols)
+    packed, scales, zeros, affine, W = matrix(rng, rows, cols, "z4")
+    w = xb.DeviceW4(packed, scales, zeros, rows, cols, affine=affine)
+    x = rng.normal(0, 1, (m, cols)).astype(np.float32)
+    x = (x * np.array([1e-34, 1e-36, 3e-38, 1e-40, 0.0, 1.0])[:, None]).astype(np.float32)
+    x64 = x.astype(np.float64)
+    weight, gate, ref = np.ones(cols, np.float32), np.ones((m, cols), np.float32), None
+    wd, gd = dev(weight), dev(gate)
+    if pro == "rms":  # eps far above the squares: x / 1e-3
+        ref = ctypes.byref(xb.Prologue(xb.PRO_RMS, 0, wd.ptr, None, 1e-6))
+        x64 = x64 / np.sqrt((x64**2).mean(-1, keepdims=True) + 1e-6)
+    elif pro == "gated":
+        ref = ctypes.byref(xb.Prologue(xb.PRO_GATED_HEAD, 128, wd.ptr, gd.ptr, 1e-6))
+        h = x64.reshape(m, -1, 128)
+        x64 = (h / np.sqrt((h**2).mean(-1, keepdims=True) + 1e-6)).reshape(m, cols) / (1 + np.exp(-1.0))
+    xd, yd = dev(x), xb.DeviceBuffer(4 * m * rows)
+    ws = xb.DeviceBuffer(xb.hip().xqhip_gemm_workspace_bytes(m, cols, rows))
+    xb.ck(xb.hip().xqhip_gemm_w4a16(w.ref, xd.ptr, m, cols, ref, cols, yd.ptr, rows, xb.EPI_STORE, ws.ptr, ws.nbytes, None))
+    got = yd.download(np.float32, m * rows).reshape(m, rows)
+    G = cols // 64
+    # a prologue's own roundings: a few of fp32 on each x, and of its subnormals (2^-149) where it ends there
+    lift = 2.0**-21 if pro != "none" else 0.0
+    tol = (2.0**-20 + lift + (8 * G + 16) * 2.0**-26) * (np.abs(x64) @ np.abs(W).T) + 2.0**-148
+    tol += 4 * 2.0**-149 * np.abs(W).sum(-1) if pro != "none" else 0.0
+    err = np.abs(got - x64 @ W.T)
+    assert (err <= tol).all(), (err / tol).max(-1)

@@ -37,6 +37,9 @@ __device__ __forceinline__ uint32_t pack_h2(_Float16 lo, _Float16 hi) {
 // ts[t] (exact).  Rows m .. m_pad - 1 are zero-filled (ts 1).
 // ---------------------------------------------------------------------------
 constexpr int kPrepMaxHeads = 256;
+// A row below 2^-114 is raised by 2^127, the largest power fp32 has: half the last fp16 bit is then 2^-152, less than
+// fp32's own smallest value.
+constexpr int kPrepMinExp = -114;
 constexpr int kXTile = 512;  // 16-byte pieces of one group of a 32-token tile
 constexpr int kXLo = 256;    // the x_lo pieces follow the x_hi ones
 
@@ -122,6 +125,7 @@ __global__ void __launch_bounds__(256) prep_x_kernel(const float* __restrict__ x
     for (int i = 0; i < nw; ++i) mx = fmaxf(mx, red[i]);
     int ex = 0;
     frexpf(mx, &ex);                                       // mx = f 2^ex, f in [0.5, 1)
+    ex = max(ex, kPrepMinExp);
     const float down = mx > 0.0f ? ldexpf(1.0f, 13 - ex) : 1.0f;  // mx * down in [2^12, 2^13)
     if (threadIdx.x == 0) ts[t] = mx > 0.0f ? ldexpf(1.0f, ex - 13) : 1.0f;
     for (int c8 = threadIdx.x; c8 < nch; c8 += blockDim.x) {
@@ -250,6 +254,7 @@ __global__ void __launch_bounds__(256) prep_x_vec_kernel(const float* __restrict
     mx = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
     int ex = 0;
     frexpf(mx, &ex);
+    ex = max(ex, kPrepMinExp);
     const float down = mx > 0.0f ? ldexpf(1.0f, 13 - ex) : 1.0f;
     if (threadIdx.x == 0) ts[t] = mx > 0.0f ? ldexpf(1.0f, ex - 13) : 1.0f;
 #pragma unroll
