@@ -128,3 +128,36 @@ def test_rows_of_tiny_values(cols, pro):
     tol += 4 * 2.0**-149 * np.abs(W).sum(-1) if pro != "none" else 0.0
     err = np.abs(got - x64 @ W.T)
     assert (err <= tol).all(), (err / tol).max(-1)
+
+
+@pytest.mark.parametrize("pro", ["none", "rms", "gated"])
+@pytest.mark.parametrize("cols", [2048, 4096, 6144, 8192, 10240, 12288, 2176])
+def test_prologues_of_each_width(cols, pro):
+    """The preparation's vectorised widths (2048 times 1 to 6) and a general one, each prologue: weights and
+    gates that differ in every column.  A prologue rounds x a few times (its sum of squares with errors of either sign),
+    silu by 4 ulp: 2^-20 of x more than without."""
+    rows, m = 64, 5
+    rng = np.random.default_rng(cols)
+    packed, scales, zeros, affine, W = matrix(rng, rows, cols, "s16")
+    w = xb.DeviceW4(packed, scales, zeros, rows, cols, affine=affine)
+    x, gate = (rng.normal(0, 1, (m, cols + 4)).astype(np.float32) for _ in range(2))
+    weight = rng.normal(1, 0.3, cols).astype(np.float32)
+    xd, gd, wd, ref = dev(x), dev(gate), dev(weight), None
+    x64, g64, w64 = x[:, :cols].astype(np.float64), gate[:, :cols].astype(np.float64), weight.astype(np.float64)
+    if pro == "rms":
+        ref = ctypes.byref(xb.Prologue(xb.PRO_RMS, 0, wd.ptr, None, 1e-6))
+        x64 = x64 / np.sqrt((x64**2).mean(-1, keepdims=True) + 1e-6) * w64
+    elif pro == "gated":
+        ref = ctypes.byref(xb.Prologue(xb.PRO_GATED_HEAD, 128, wd.ptr, gd.ptr, 1e-6))
+        h = x64.reshape(m, -1, 128)
+        h = h / np.sqrt((h**2).mean(-1, keepdims=True) + 1e-6) * w64[:128]
+        x64 = h.reshape(m, cols) * g64 / (1 + np.exp(-g64))
+    yd = xb.DeviceBuffer(4 * m * rows)
+    ws = xb.DeviceBuffer(xb.hip().xqhip_gemm_workspace_bytes(m, cols, rows))
+    xb.ck(xb.hip().xqhip_gemm_w4a16(w.ref, xd.ptr, m, cols + 4, ref, cols + 4, yd.ptr, rows, xb.EPI_STORE, ws.ptr,
+                                    ws.nbytes, None))
+    got = yd.download(np.float32, m * rows).reshape(m, rows)
+    G = cols // 64
+    tol = (2.0**-20 + (2.0**-20 if pro != "none" else 0.0) + (8 * G + 16) * 2.0**-26) * (np.abs(x64) @ np.abs(W).T)
+    err = np.abs(got - x64 @ W.T)
+    assert (err <= tol).all(), (err / tol).max()
