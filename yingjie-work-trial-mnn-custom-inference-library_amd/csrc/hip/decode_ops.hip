@@ -1198,8 +1198,8 @@ __global__ void __launch_bounds__(kHeadThreads) attn_decode_part_kernel(AttnDeco
 // attn_decode_part_kernel's without the counter, its record [kWideStride] of the
 // workspace merged by attn_merge_kernel after the kernel boundary.  One block
 // per CU: 16 query heads in 16 splits.  What bounds it: a block's serial chain (q and
-// k prepared, scores, maximum, exp, value sum) and the merge's launch.  16 / 4 heads, 2000 positions: 6.9 + 3.7 us for the merge, against
-// 19.6 us in all for a block per (kv head, 31 positions) that took its four query heads in turn.
+// k prepared, scores, maximum, exp, value sum) and the merge's launch.  16 / 4 heads, 2000 positions: 7.7 us for both,
+// against 19.1 for a block per (kv head, 31 positions) that took its four query heads in turn.
 constexpr int kWideHd = 256, kWideMaxSplits = 32;
 constexpr int kWideStride = 288;  // floats per record: m, l, 2 pad, o[256], pad to whole 128-byte lines
 static_assert(kWideMaxSplits * kWideStride <= kAttnMaxSlots * (kWideHd + 2), "the slot workspace holds the records");
@@ -1225,31 +1225,27 @@ __global__ void __launch_bounds__(kHeadThreads) attn_decode_wide_kernel(AttnDeco
     else head_attention<kWideHd, kPassSubs<kWideHd, true>, true>(a, sm, pos, c0, c1, fresh, out);
 }
 
+// A lane of each wave holds one split's (m, l), so a weight is one exp and reaches the others as a scalar, where every
+// thread took all of them before: 4 / 4 heads, 30 positions, both launches 7.8 us, 10.7 before; 16 / 4 heads, 2000
+// positions 7.7, 8.6 before.
 template <int MAXS>
 __global__ void __launch_bounds__(kWideHd) attn_merge_kernel(GqaLaunch p, const float* part, int splits) {
-    const int qh = blockIdx.x, d = threadIdx.x;
+    static_assert(MAXS <= kWave, "a lane per split");
+    const int qh = blockIdx.x, d = threadIdx.x, lane = threadIdx.x & (kWave - 1);
     // no gate projection: the reference's zero gate, sigmoid(0) (custom_model.cpp:750-753)
     const float g = p.gate ? p.gate[static_cast<size_t>(qh) * p.gate_stride + d] : 0.0f;
-    float mv[MAXS], lv[MAXS], ov[MAXS], M = -INFINITY;
+    auto record = [&](int s) { return part + (static_cast<size_t>(min(s, splits - 1)) * p.nq + qh) * kWideStride; };
+    const float ms = record(lane)[0], ls = record(lane)[1];
+    float ov[MAXS];
 #pragma unroll
-    for (int s = 0; s < MAXS; ++s) {  // past the last split: its record again, weight 0 (every load in flight)
-        const float* q = part + (static_cast<size_t>(min(s, splits - 1)) * p.nq + qh) * kWideStride;
-        mv[s] = q[0];
-        lv[s] = q[1];
-        ov[s] = q[kAttnPartO + d];
-    }
+    for (int s = 0; s < MAXS; ++s) ov[s] = record(s)[kAttnPartO + d];  // past the last split: its again, weight 0
+    const float m = lane < splits ? ms : -INFINITY;
+    const float w = expf(m - wave_max(m));  // an empty range (m = -inf): 0
+    const float L = wave_sum(w * ls);
+    float acc = 0.0f;
 #pragma unroll
-    for (int s = 0; s < MAXS; ++s) {
-        if (s >= splits) mv[s] = -INFINITY;
-        M = fmaxf(M, mv[s]);
-    }
-    float L = 0.0f, acc = 0.0f;
-#pragma unroll
-    for (int s = 0; s < MAXS; ++s) {
-        const float w = expf(mv[s] - M);  // an empty range (m = -inf): 0
-        L += w * lv[s];
-        acc += w * ov[s];
-    }
+    for (int s = 0; s < MAXS; ++s)
+        acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s)) * ov[s];
     p.out[static_cast<size_t>(qh) * kWideHd + d] = (acc * (1.0f / L)) * sigmoid_dev(g);
 }
 
