@@ -149,9 +149,9 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillAttnLaunch p) 
 //
 // Measured: 512 tokens after 3584, 32 / 8 heads of 128: 76 us (the kernel
 // before, one wave per query head of 16 tokens with no key split, 181 us);
-// 16 tokens after 0: 7.5 us (9.1; 10.7 with q in operand order and all eight
-// waves merged); 333 tokens after 512, 16 / 4 heads of 256: 41 us
-// (prefill_attn_kernel 3603 us).
+// 16 tokens after 0: 7.4 us (9.2; 10.7 with q in operand order and all eight
+// waves merged); 333 tokens after 512, 16 / 4 heads of 256: 36.6 us
+// (prefill_attn_kernel 3595 us).
 constexpr int kFTile = 32;  // keys and columns of an MFMA tile
 
 template <int HD, int CT, int KS>
@@ -259,6 +259,9 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
         }
     }
     load(p.k_cache, 0, kr);
+    // 256 dims: the first values with the first keys, one round trip less for a short context (2 tokens after 0: 11.0
+    // us, 12.5 without and with the last keys' stores).  128 dims have 8 us there and lose 10 % on long ones.
+    if constexpr (HD > 128) load(p.v_cache, 0, vr);
     float* Ql = reinterpret_cast<float*>(Vl);  // [kCols][kLdo]
 #pragma unroll
     for (int u = 0; u < F::kPasses; ++u)
@@ -305,7 +308,7 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
 #pragma unroll
     for (int j = 0; j < kDimTiles; ++j) o[j] = floatx16{};
     for (int c0 = 0; c0 <= last; c0 += F::kKeys) {  // block-uniform
-        load(p.v_cache, c0, vr);
+        if (HD <= 128 || c0 > 0) load(p.v_cache, c0, vr);
         const int key0 = c0 + ks * kFTile;
         const bool any = key0 <= last;  // wave-uniform: this wave's tile holds a key
         half8 phi[2], plo[2];
@@ -351,9 +354,10 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
             }
         }
         store(Vl, F::kLdv, vr);
-        // block-uniform; 256 dims load on (past `last`: nothing is read): the branch costs them spilled registers
-        const bool more = HD > 128 || c0 + F::kKeys <= last;
-        if (more) load(p.k_cache, c0 + F::kKeys, kr);
+        // block-uniform; 256 dims load on (past `last`: nothing is read): a branch around the loads costs them spilled
+        // registers, one around the stores below none
+        const bool more = c0 + F::kKeys <= last;
+        if (HD > 128 || more) load(p.k_cache, c0 + F::kKeys, kr);
         __syncthreads();  // V is staged; every wave has read K
         if (any) {
             // transposed reads: 16 lanes cover four keys x 16 dims, lane i gets dim i of the four
