@@ -259,8 +259,8 @@ __global__ void __launch_bounds__(kWave * CT * KS, (CT * KS + 3) / 4) prefill_at
         }
     }
     load(p.k_cache, 0, kr);
-    // 256 dims: the first values with the first keys, one round trip less for a short context (2 tokens after 0: 11.0
-    // us, 12.5 without and with the last keys' stores).  128 dims have 8 us there and lose 10 % on long ones.
+    // 256 dims: the first values with the first keys, one round trip less for a short context (16 / 4 heads, 2 tokens
+    // after 0: 11.2 us, 12.5 without).  128 dims gain nothing there (7.5, 7.3 without) and lose 10 % on long contexts.
     if constexpr (HD > 128) load(p.v_cache, 0, vr);
     float* Ql = reinterpret_cast<float*>(Vl);  // [kCols][kLdo]
 #pragma unroll
