@@ -331,7 +331,7 @@ def time_prefill_gemm(rows=24576, cols=4096, m=512, n=20):
     w.free()
     flop = 2.0 * m * rows * cols
     tflops = flop / (us * 1e-6) / 1e12
-    return {"bound": "mfma", "kernel": "prep_x_vec_kernel + gemm_w4_mfma_kernel<4, 1, 2, 4, 2, 2>: prefill gate/up "
+    return {"bound": "mfma", "kernel": "prep_x_vec_kernel + gemm_w4_mfma_kernel<4, 1, 2, 2, 2, 2>: prefill gate/up "
                                        f"{rows}x{cols} W4A16 g64 over {m} tokens, RMSNorm prologue, SiLU*up epilogue",
             "method": f"HIP events around {n} back-to-back calls of xqhip_gemm_w4a16 (preparation + GEMM); "
                       "algorithmic FLOP = 2 m rows cols",

@@ -331,13 +331,11 @@ static bool prep_vec_ok(const GemmLaunch& p) {
 // fp16 subtractions.  The LDS reads, the unpacking and the scaling of a finished
 // group's sums are placed between the MFMAs.
 //
-// What bounds it: the MFMAs' power.  A loop of nothing but these MFMAs on
-// random operands runs at 1.35 PFLOP/s (2.2 on zeros), like a large library
-// product in fp16; gate/up (24576x4096, 512 tokens) issues 206 GFLOP in 186 us =
-// 1.1 PFLOP/s.  Leaving out the unpacking, the scaling, the barriers or the LDS
-// reads (timing only) changes it by at most 5 %.  The kernel before (weights as
-// the row operand, 32-row waves that each read every token's fragments, x staged
-// through registers) took 255 us.
+// What bounds it: the MFMAs, at the clock that their power leaves.  gate/up (24576x4096, 512 tokens) issues 206 GFLOP in
+// 188 us = 1.1 PFLOP/s, the matrix cores busy for 58 % of the cycles at 1.8 GHz (the card's clock is 2.4); a loop of
+// nothing but these MFMAs on random operands runs at 1.35 PFLOP/s (2.2 on zeros).  Leaving out the unpacking, the
+// scaling, the barriers or the LDS reads (timing only) changes it by at most 5 %.  The kernel before (weights as
+// the row operand, 32-row waves that each read every token's fragments, x staged through registers) took 255 us.
 // ---------------------------------------------------------------------------
 constexpr int kGemmPad = 128;  // tokens are padded to at most a multiple of this
 constexpr int kGemmMaxSplits = 8;
